@@ -768,10 +768,10 @@ void build_neighbours(fjsph_ctx* ctx, bool reorder)
         }
         const int32_t mc = ctx->sc_host->max_count;
         ctx->max_count = mc;
-        if (mc <= ctx->nl.cap) break;
+        if (mc <= ctx->nl.cap && ctx->nl.lu4) break;
         /* capacity in entries, a multiple of the 4-entry batch */
         const int32_t cap = ((mc + mc / 8 + 8) + 7) / 8 * 8;
-        dalloc(ctx->nl.lu4, size_t(cap / 4) * ctx->nl.npad);
+        dalloc(ctx->nl.lu4, size_t(cap / 4 + kRowSlack) * ctx->nl.npad + kTargetSlack);
         ctx->nl.cap = cap;
     }
     if (ctx->max_count > ctx->nl.cap) throw std::string("neighbour list capacity could not be established");

@@ -194,35 +194,44 @@ __device__ __forceinline__ void split_rel(double x, double ref, float& hi, float
 /* ------------------------------------------------------------ list rows */
 
 /* Lock-step walk of one target's rows: `row` advances in every lane of the
- * wave together; the next row is in flight while the current one is used.
- * Rows past nrows read as all-NO_ENTRY.  Every lane with a list walks it,
- * also a lane whose target the pass does not compute (`on` false): the
- * build pads each tile's rows to the wave's largest count, and the wave
- * leaves a tile only when no lane has an entry of it left, so a lane that
- * dropped out could leave the others on padding rows of the tile. */
+ * wave together.  take() hands out the current row and asks for the next
+ * one, so the load is in flight while the row's pairs run (a load issued
+ * after them, at the end of the loop, was waited for at once: the loop
+ * carries it in a register, and the copy into that register needs the
+ * value).  The load has no branch: a lane reads on past its own nrows (the
+ * array has kRowSlack rows and a block of targets to spare) and row_in()
+ * tells what counts.  Every lane with a list walks it, also a lane whose
+ * target the pass does not compute (`on` false): the build pads each tile's
+ * rows to the wave's largest count, and the wave leaves a tile only when no
+ * lane has an entry of it left, so a lane that dropped out could leave the
+ * others on padding rows of the tile. */
 struct Rows {
-    const uint64_t* rp; /* the next row (row nxt of the target) */
+    const uint64_t* rp; /* the next row, at position 0 */
     int64_t stride;
-    int nxt, nrows;
+    uint32_t p;
+    int row, nrows;
     bool on;
-    uint64_t u, un;
-    __device__ __forceinline__ void init(const NbrList& nl, int64_t p, int nrows_, bool on_)
+    uint64_t u;
+    __device__ __forceinline__ void init(const NbrList& nl, int p_, int nrows_, bool on_)
     {
         on = on_;
         nrows = nrows_;
         stride = nl.npad;
-        rp = nl.lu4 + p;
-        u = nrows > 0 ? *rp : ~0ull;
-        rp += stride;
-        nxt = 1;
-        un = nrows > 1 ? *rp : ~0ull;
+        p = uint32_t(p_);
+        row = 0;
+        u = nl.lu4[p];
+        rp = nl.lu4 + stride;
     }
-    __device__ __forceinline__ void advance(const NbrList&)
+    /* the current row is one of the lane's and lies in the tile that ends
+     * below `top` */
+    __device__ __forceinline__ bool row_in(uint32_t top) const { return row < nrows && (uint32_t(u) & 0xFFFFu) < top; }
+    __device__ __forceinline__ uint64_t take()
     {
-        u = un;
+        const uint64_t cur = u;
+        u = rp[p];
         rp += stride;
-        ++nxt;
-        un = nxt < nrows ? *rp : ~0ull;
+        ++row;
+        return cur;
     }
 };
 
@@ -237,10 +246,10 @@ struct Rows {
  * per-lane accumulator arrays stay in registers. */
 #define FJ_TILE_ENTRIES_BEGIN(cu, nl, base)                                               \
     for (;;) {                                                                            \
-        const bool fj_act = (uint32_t((cu).u) & 0xFFFFu) < uint32_t((base) + TILE);        \
+        const bool fj_act = (cu).row_in(uint32_t((base) + TILE));                         \
         if (!__any(fj_act)) break;                                                        \
+        uint64_t fj_u = (cu).take();                                                      \
         if (fj_act && (cu).on) {                                                          \
-            uint64_t fj_u = (cu).u;                                                       \
             _Pragma("unroll 1") for (int fj_q = 0; fj_q < 4; ++fj_q)                     \
             {                                                                             \
                 const uint32_t fj_uq = uint32_t(fj_u) & 0xFFFFu;                          \
@@ -251,8 +260,49 @@ struct Rows {
 #define FJ_TILE_ENTRIES_END(cu, nl) \
             }                       \
         }                           \
-        (cu).advance(nl);           \
     }
+
+/* FJ_TILE_PAIRS_BEGIN(cu, nl, base, P) { body } FJ_TILE_PAIRS_END(cu, nl):
+ * the same walk, P (1, 2 or 4) entries of a row at a time and without a
+ * branch per entry: `t[e]` is the tile-local index of entry e and `ok[e]`
+ * whether there is one (t[e] = 0, a staged slot, otherwise), so the body can
+ * read the P records before it uses the first of them and masks the terms of
+ * a missing entry itself (its record may lie far outside the support: r is
+ * taken as 0, where every factor of a pair is finite).  Entries fill a row
+ * from its low end. */
+#define FJ_TILE_PAIRS_BEGIN(cu, nl, base, P)                                              \
+    for (;;) {                                                                            \
+        const bool fj_act = (cu).row_in(uint32_t((base) + TILE));                         \
+        if (!__any(fj_act)) break;                                                        \
+        uint64_t fj_u = (cu).take();                                                      \
+        if (!(fj_act && (cu).on)) fj_u = ~0ull;                                           \
+        _Pragma("unroll 1") for (int fj_q = 0; fj_q < 4; fj_q += (P))                     \
+        {                                                                                 \
+            int t[P];                                                                     \
+            bool ok[P];                                                                   \
+            _Pragma("unroll") for (int e = 0; e < (P); ++e)                               \
+            {                                                                             \
+                const uint32_t fj_uq = uint32_t(fj_u >> (16 * e)) & 0xFFFFu;              \
+                ok[e] = fj_uq != NO_ENTRY;                                                \
+                t[e] = ok[e] ? int(fj_uq) - (base) : 0;                                   \
+            }                                                                             \
+            if (!__any(ok[0])) break;                                                     \
+            fj_u = (P) < 4 ? fj_u >> (16 * ((P) & 3)) : ~0ull;
+
+#define FJ_TILE_PAIRS_END(cu, nl) \
+        }                         \
+    }
+
+/* Entries of a row taken together in the mixed-precision passes.  The pair
+ * loops wait on LDS more than they compute (0.56-0.9 vector instructions per
+ * CU-cycle at 4-5 waves per SIMD): with the records of two entries asked for
+ * at once and the next row loaded while the current one runs, at 1M particles
+ * dSPH 1.02 -> 0.86 ms a launch, surface loop 1 with loops 2-3 and shift
+ * 2.44 -> 2.09, the ALE force 0.88 -> 0.79; one entry at a time 0.88, 2.22,
+ * 0.80; four spill at 5 waves per SIMD (0.95, 4.7, 2.2).  The force pass
+ * without ALE reads less per pair and does better one at a time (268k
+ * particles: 0.432 -> 0.403 ms, 0.417 with two). */
+constexpr int kPairs = 2;
 
 __device__ __forceinline__ int wave_max(int v)
 {
@@ -783,14 +833,24 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
             }
             ts.load(tg, h, tk + 1, NT, U);
             __syncthreads();
-            FJ_TILE_ENTRIES_BEGIN(cu, nl, base)
-                const float4 A = tA[t];
+            FJ_TILE_PAIRS_BEGIN(cu, nl, base, kPairs)
+                float4 Ae[kPairs], Xe[kPairs];
+                float Re[kPairs];
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                    Ae[e] = tA[t[e]];
+                    Re[e] = tR[t[e]];
+                    if constexpr (FR) Xe[e] = tX[t[e]];
+                }
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                const float4 A = Ae[e];
                 const float pj[3] = {A.x, A.y, A.z};
                 float Rji[D], rr;
 #pragma unroll
                 for (int a = 0; a < D; ++a) Rji[a] = (pj[a] - xit[a]) - xlo[a];
                 if constexpr (FR) {
-                    const float4 X = tX[FR ? t : 0];
+                    const float4 X = Xe[e];
                     const float xbj[3] = {X.x, X.y, X.z};
                     float Rb[D];
 #pragma unroll
@@ -803,15 +863,17 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
 #pragma unroll
                     for (int a = 1; a < D; ++a) rr += Rji[a] * Rji[a];
                 }
+                if (!ok[e]) rr = 0.f;
                 float W, fg;
                 wendland<float>(fast_sqrt<float>(rr), Ht, inv_Hf, Wcf, W, fg);
-                const bool nb = A.w > 0.f;
-                const float volj = fabsf(A.w);
+                const float sv = ok[e] ? A.w : 0.f;
+                const bool nb = sv > 0.f;
+                const float volj = fabsf(sv);
                 const float nbf = nb ? 1.f : 0.f;
                 float G[D];
 #pragma unroll
                 for (int a = 0; a < D; ++a) G[a] = -fg * Rji[a];
-                const float drho = volj * ((tR[t] - drhoi) - rlo);
+                const float drho = volj * ((Re[e] - drhoi) - rlo);
                 int k = 0;
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
@@ -827,7 +889,8 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
                 }
                 fks += nbf * W;
                 fcol += nbf * volj * W;
-            FJ_TILE_ENTRIES_END(cu, nl)
+                }
+            FJ_TILE_PAIRS_END(cu, nl)
             /* the tile's FP32 partial sums into the FP64 totals */
 #pragma unroll
             for (int k = 0; k < NS; ++k) {
@@ -1394,14 +1457,28 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
             }
             ts.load(tg, h, tk + 1, NT, U);
             __syncthreads();
-            FJ_TILE_ENTRIES_BEGIN(cu, nl, base)
-                const float4 A = tA[t];
+            FJ_TILE_PAIRS_BEGIN(cu, nl, base, kPairs)
+                float4 Ae[kPairs], Be[kPairs], Ge[kPairs], Xe[kPairs];
+                float2 Ee[kPairs];
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                    Ae[e] = tA[t[e]];
+                    Be[e] = tB[t[e]];
+                    if constexpr (with_diss) {
+                        Ge[e] = tG[t[e]];
+                        Ee[e] = tE[t[e]];
+                    }
+                    if constexpr (FR) Xe[e] = tX[t[e]];
+                }
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                const float4 A = Ae[e];
                 const float pj[3] = {A.x, A.y, A.z};
                 float Rji[D], rr;
 #pragma unroll
                 for (int a = 0; a < D; ++a) Rji[a] = (pj[a] - xit[a]) - xlo[a];
                 if constexpr (FR) {
-                    const float4 X = tX[FR ? t : 0];
+                    const float4 X = Xe[e];
                     const float xbj[3] = {X.x, X.y, X.z};
                     float Rb[D];
 #pragma unroll
@@ -1414,12 +1491,14 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
 #pragma unroll
                     for (int a = 1; a < D; ++a) rr += Rji[a] * Rji[a];
                 }
+                if (!ok[e]) rr = 0.f;
                 const float r = fast_sqrt<float>(rr);
                 float W, fg;
                 wendland<float>(r, Ht, inv_H, Wc, W, fg);
-                const float4 B = tB[t];
+                const float4 B = Be[e];
+                const float volj = ok[e] ? A.w : 0.f;
                 if constexpr (with_surf) {
-                    if (testing && !found) {
+                    if (testing && !found && ok[e]) {
                         /* point-T test (src/Geometry.cpp:43-98) in FP32 unless
                          * within the margin of a threshold */
                         float xjT[D];
@@ -1456,18 +1535,18 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
                         else {
                             /* rare: the slot goes straight to memory */
                             if (npend < kSurfPendMax)
-                                reinterpret_cast<int32_t*>(ax.spend)[i * kSurfPendMax + npend] = tsl[with_surf ? t : 0];
+                                reinterpret_cast<int32_t*>(ax.spend)[i * kSurfPendMax + npend] = tsl[with_surf ? t[e] : 0];
                             ++npend;
                         }
                     }
-                    const float f = A.w * (high ? (B.w - lamf) : B.w) * fg;
+                    const float f = volj * (high ? (B.w - lamf) : B.w) * fg;
 #pragma unroll
                     for (int a = 0; a < D; ++a) fnrm[a] -= f * Rji[a];
                 }
                 if constexpr (with_diss) {
                     /* dissipation_terms pair term (src/Shifting.cpp:141-173) */
-                    const float4 G = tG[t];
-                    const float2 E = tE[t];
+                    const float4 G = Ge[e];
+                    const float2 E = Ee[e];
                     const float vj[3] = {B.x, B.y, B.z}, grj[3] = {G.x, G.y, G.z};
                     float g[D];
 #pragma unroll
@@ -1477,7 +1556,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
 #pragma unroll
                     for (int a = 1; a < D; ++a) rdotg += Rji[a] * g[a];
                     const float drho = (G.w - drhoi) - rlo;
-                    if (E.y > 0.f) {
+                    if (ok[e] && E.y > 0.f) {
                         float vdotr = ((vj[0] - vit[0]) - vlo[0]) * Rji[0];
 #pragma unroll
                         for (int a = 1; a < D; ++a) vdotr += ((vj[a] - vit[a]) - vlo[a]) * Rji[a];
@@ -1492,12 +1571,13 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
                         float gsum = (gri[0] + grj[0]) * Rji[0];
 #pragma unroll
                         for (int a = 1; a < D; ++a) gsum += (gri[a] + grj[a]) * Rji[a];
-                        frd += A.w * (drho + 0.5f * gsum) * rdotg * idist2;
+                        frd += volj * (drho + 0.5f * gsum) * rdotg * idist2;
                     } else {
-                        frd += A.w * drho * rdotg * idist2;
+                        frd += volj * drho * rdotg * idist2;
                     }
                 }
-            FJ_TILE_ENTRIES_END(cu, nl)
+                }
+            FJ_TILE_PAIRS_END(cu, nl)
 #pragma unroll
             for (int a = 0; a < D; ++a) {
                 nrm[a] += double(fnrm[a]);
@@ -1801,14 +1881,23 @@ __global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevSt
             }
             ts.load(tg, h, tk + 1, NT, U);
             __syncthreads();
-            FJ_TILE_ENTRIES_BEGIN(cu, nl, base)
-                const float4 A = tA[t], N = tN[t];
+            FJ_TILE_PAIRS_BEGIN(cu, nl, base, kPairs)
+                float4 Ae[kPairs], Ne[kPairs], Xe[kPairs];
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                    Ae[e] = tA[t[e]];
+                    Ne[e] = tN[t[e]];
+                    if constexpr (FR) Xe[e] = tX[t[e]];
+                }
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                const float4 A = Ae[e], N = Ne[e];
                 const float pj[3] = {A.x, A.y, A.z}, nj[3] = {N.x, N.y, N.z};
                 float Rij[D], rr;
 #pragma unroll
                 for (int a = 0; a < D; ++a) Rij[a] = (pj[a] - xit[a]) - xlo[a];
                 if constexpr (FR) {
-                    const float4 X = tX[FR ? t : 0];
+                    const float4 X = Xe[e];
                     const float xbj[3] = {X.x, X.y, X.z};
                     float Rb[D];
 #pragma unroll
@@ -1825,7 +1914,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevSt
                 bool nj_nz = false;
 #pragma unroll
                 for (int a = 0; a < D; ++a) nj_nz = nj_nz || nj[a] != 0.f;
-                if (ni_nz && nj_nz) {
+                if (ok[e] && ni_nz && nj_nz) {
                     float W, fg;
                     wendland<float>(r, Ht, inv_Hf, Wcf, W, fg);
                     float tt = 0.f;
@@ -1838,15 +1927,16 @@ __global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevSt
                     }
                     fcurve += A.w * tt;
                 }
-                if (occl) {
+                if (ok[e] && occl) {
                     float q = Rij[0] * Vd[0];
 #pragma unroll
                     for (int a = 1; a < D; ++a) q += Rij[a] * Vd[a];
                     q = -q / r;
                     if (q > qmax) qmax = q;
                 }
-                zone = zone || N.w != 0.f;
-            FJ_TILE_ENTRIES_END(cu, nl)
+                zone = zone || (ok[e] && N.w != 0.f);
+                }
+            FJ_TILE_PAIRS_END(cu, nl)
             curve += double(fcurve);
             fcurve = 0.f;
         }
@@ -2099,14 +2189,23 @@ __global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState
             }
             ts.load(tg, h, tk + 1, NT, U);
             __syncthreads();
-            FJ_TILE_ENTRIES_BEGIN(cu, nl, base)
-                const float4 A = tA[t], V = tV[t];
+            FJ_TILE_PAIRS_BEGIN(cu, nl, base, kPairs)
+                float4 Ae[kPairs], Ve[kPairs], Xe[kPairs];
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                    Ae[e] = tA[t[e]];
+                    Ve[e] = tV[t[e]];
+                    if constexpr (FR) Xe[e] = tX[t[e]];
+                }
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                const float4 A = Ae[e], V = Ve[e];
                 const float pj[3] = {A.x, A.y, A.z}, vj[3] = {V.x, V.y, V.z};
                 float Rji[D], rr;
 #pragma unroll
                 for (int a = 0; a < D; ++a) Rji[a] = (pj[a] - xit[a]) - xlo[a];
                 if constexpr (FR) {
-                    const float4 X = tX[FR ? t : 0];
+                    const float4 X = Xe[e];
                     const float xbj[3] = {X.x, X.y, X.z};
                     float Rb[D];
 #pragma unroll
@@ -2119,11 +2218,12 @@ __global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState
 #pragma unroll
                     for (int a = 1; a < D; ++a) rr += Rji[a] * Rji[a];
                 }
+                if (!ok[e]) rr = 0.f;
                 float W, fg;
                 wendland<float>(fast_sqrt<float>(rr), Ht, inv_Hf, Wcf, W, fg);
                 const float w = W * inv_Wdx;
                 const float w2 = w * w;
-                const float f = (1.f + 0.2f * (w2 * w2)) * fg * fabsf(A.w);
+                const float f = (1.f + 0.2f * (w2 * w2)) * fg * (ok[e] ? fabsf(A.w) : 0.f);
                 float dv2 = 0.f;
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
@@ -2131,14 +2231,15 @@ __global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState
                     const float dv = (vj[a] - vit[a]) - vlo[a];
                     dv2 += dv * dv;
                 }
-                if (A.w > 0.f) {
+                if (ok[e] && A.w > 0.f) {
                     double d = 0.0;
 #pragma unroll
-                    for (int a = 0; a < D; ++a) d += nhat[a] * tn[a][t];
+                    for (int a = 0; a < D; ++a) d += nhat[a] * tn[a][t[e]];
                     if (d >= -1.0 && d <= 1.0 && d < dmin) dmin = d;
                 }
-                maxU2 = fmaxf(maxU2, dv2);
-            FJ_TILE_ENTRIES_END(cu, nl)
+                maxU2 = fmaxf(maxU2, ok[e] ? dv2 : 0.f);
+                }
+            FJ_TILE_PAIRS_END(cu, nl)
 #pragma unroll
             for (int a = 0; a < D; ++a) {
                 du[a] += double(fdu[a]);
@@ -2293,15 +2394,26 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
             }
             ts.load(tg, h, tk + 1, NT, U);
             __syncthreads();
-            FJ_TILE_ENTRIES_BEGIN(cu, nl, base)
-                const float4 A = tA[t], N = tN[t];
+            FJ_TILE_PAIRS_BEGIN(cu, nl, base, kPairs)
+                float4 Ae[kPairs], Ne[kPairs], Ve[kPairs], Xe[kPairs];
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                    Ae[e] = tA[t[e]];
+                    Ne[e] = tN[t[e]];
+                    Ve[e] = tV[t[e]];
+                    if constexpr (FR) Xe[e] = tX[t[e]];
+                }
+#pragma unroll
+                for (int e = 0; e < kPairs; ++e) {
+                const float4 A = Ae[e], N = Ne[e];
                 const float pj[3] = {A.x, A.y, A.z}, nj[3] = {N.x, N.y, N.z};
-                const float volj = fabsf(A.w);
+                const float sv = ok[e] ? A.w : 0.f;
+                const float volj = fabsf(sv);
                 float Rij[D], rr;
 #pragma unroll
                 for (int a = 0; a < D; ++a) Rij[a] = (pj[a] - xit[a]) - xlo[a];
                 if constexpr (FR) {
-                    const float4 X = tX[FR ? t : 0];
+                    const float4 X = Xe[e];
                     const float xbj[3] = {X.x, X.y, X.z};
                     float Rb[D];
 #pragma unroll
@@ -2314,6 +2426,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
 #pragma unroll
                     for (int a = 1; a < D; ++a) rr += Rij[a] * Rij[a];
                 }
+                if (!ok[e]) rr = 0.f;
                 const float r = fast_sqrt<float>(rr);
                 float W, fg;
                 wendland<float>(r, Ht, inv_Hf, Wcf, W, fg);
@@ -2332,7 +2445,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
                     }
                     fcurve += volj * tt;
                 }
-                if (occl) {
+                if (ok[e] && occl) {
                     /* -R_ij . Vd / r with the hardware reciprocal (1 ulp) in
                      * place of the IEEE division */
                     float q = Rij[0] * Vd[0];
@@ -2341,10 +2454,10 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
                     q = -q * fast_rcp<float>(r);
                     if (q > qmax) qmax = q;
                 }
-                zone = zone || N.w != 0.f;
+                zone = zone || (ok[e] && N.w != 0.f);
                 /* particle_shift */
                 if (work) {
-                    const float4 V = tV[t];
+                    const float4 V = Ve[e];
                     const float vj[3] = {V.x, V.y, V.z};
                     const float w = W * inv_Wdx;
                     const float w2 = w * w;
@@ -2356,23 +2469,24 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
                         const float dv = (vj[a] - vit[a]) - vlo[a];
                         dv2 += dv * dv;
                     }
-                    if (A.w > 0.f && !wide) {
+                    if (sv > 0.f && !wide) {
                         float d = ni[0] * nj[0];
 #pragma unroll
                         for (int a = 1; a < D; ++a) d += ni[a] * nj[a];
                         if (d >= ang_yes_lo && d <= ang_yes_hi) wide = true;
                         else if (!(d >= ang_no)) {
                             /* rare: within the margin of cos(pi/12) or -1 */
-                            const int32_t sl = tsl[t];
+                            const int32_t sl = tsl[t[e]];
                             double d64 = 0.0;
 #pragma unroll
                             for (int a = 0; a < D; ++a) d64 += nhat[a] * ax.nhat[(int64_t)sl * D + a];
                             if (d64 >= -1.0 && d64 <= 1.0 && acos(d64) >= kPi / 12.0) wide = true;
                         }
                     }
-                    maxU2 = fmaxf(maxU2, dv2);
+                    maxU2 = fmaxf(maxU2, ok[e] ? dv2 : 0.f);
                 }
-            FJ_TILE_ENTRIES_END(cu, nl)
+                }
+            FJ_TILE_PAIRS_END(cu, nl)
             curve += double(fcurve);
             fcurve = 0.f;
 #pragma unroll
@@ -2961,6 +3075,7 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
                                                               const int32_t* __restrict__ part_id, TileGrid tg,
                                                               NbrList nl, const DevScalars* sc)
 {
+    constexpr int P = ALE ? kPairs : 1; /* entries taken together (kPairs) */
     __shared__ ForceTileM<ALE> ft;
     __shared__ BlockHead h;
     block_head<D>(tg, h);
@@ -3048,8 +3163,18 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
             ts.load(tg, h, tk + 1, NT, U);
             __syncthreads();
             float fa[3] = {0.f, 0.f, 0.f}, fS[3] = {0.f, 0.f, 0.f}, fr = 0.f, frc = 0.f;
-            FJ_TILE_ENTRIES_BEGIN(cu, nl, base)
-                const float4 A = ft.A[t], B = ft.B[t], X = ft.X[t];
+            FJ_TILE_PAIRS_BEGIN(cu, nl, base, P)
+                float4 Ae[P], Be[P], Xe[P], Ee[P];
+#pragma unroll
+                for (int e = 0; e < P; ++e) {
+                    Ae[e] = ft.A[t[e]];
+                    Be[e] = ft.B[t[e]];
+                    Xe[e] = ft.X[t[e]];
+                    if constexpr (ALE) Ee[e] = ft.E[t[e]];
+                }
+#pragma unroll
+                for (int e = 0; e < P; ++e) {
+                const float4 A = Ae[e], B = Be[e], X = Xe[e];
                 const float pj[3] = {A.x, A.y, A.z}, vj[3] = {B.x, B.y, B.z}, xbj[3] = {X.x, X.y, X.z};
                 float Rji[D], Vji[D];
 #pragma unroll
@@ -3070,8 +3195,9 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
 #pragma unroll
                     for (int a = 1; a < D; ++a) rr += Rji[a] * Rji[a];
                 }
+                if (!ok[e]) rr = 0.f;
                 const float r = fast_sqrt<float>(rr);
-                const float msg = A.w, Pj = B.w, irj = X.w;
+                const float msg = ok[e] ? A.w : 0.f, Pj = B.w, irj = X.w;
                 const bool bound_j = msg < 0.f;
                 const float mj = fabsf(msg);
                 const float volj = mj * irj;
@@ -3107,7 +3233,7 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
                  * skip; without ALE every fluid target has it and the terms
                  * join the momentum sum below */
                 float sf = 0.f;
-                if (st_on) {
+                if (ok[e] && st_on) {
                     const float fac = (bound_i || bound_j) ? contang_fac : 1.f;
                     sf = stm * fac * fast_cos<float>(pi3o4H * r) * fast_rcp<float>(r);
                     if constexpr (ALE) {
@@ -3116,7 +3242,7 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
                     }
                 }
                 if constexpr (ALE) {
-                    const float4 E = ft.E[t];
+                    const float4 E = Ee[e];
                     const float vpj[3] = {E.x, E.y, E.z};
                     float aj = vpj[0] * g[0];
 #pragma unroll
@@ -3136,7 +3262,8 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
 #pragma unroll
                     for (int a = 0; a < D; ++a) fa[a] += vf * Vji[a] + sf * Rji[a] - pc * g[a];
                 }
-            FJ_TILE_ENTRIES_END(cu, nl)
+                }
+            FJ_TILE_PAIRS_END(cu, nl)
 #pragma unroll
             for (int a = 0; a < D; ++a) acc[a] += double(fa[a]);
             Rrho_ -= double(fr);

@@ -1,0 +1,78 @@
+"""List walks at the edges of their rows: isolated clusters of k particles, so
+that every target has k - 1 neighbours (no row at all, rows of one to four
+entries, a second row with one) and the waves mix lanes with and without
+entries.  Pair sums against the oracle; FP64 to summation order, mixed to the
+FP32 pair terms (as test_gpu_parity.py)."""
+import numpy as np
+import pytest
+
+from fjsph_amd import abi, cases
+from tests.parity import assert_close, same_neighbour_sets
+from tests.test_gpu_parity import FP64_PASS, MIXED_STEP, _engine, _oracle
+
+pytestmark = pytest.mark.gpu
+
+SIZES = (1, 2, 3, 4, 5, 6, 8, 9, 13)
+
+
+def _clusters(dim, sizes, precision, ale):
+    dx = 1e-3
+    c = cases.fluid_block(dim, 2, dx=dx, precision=precision, H_fac=2.0, sig=0.07)
+    s = c.settings
+    s.ale = ale
+    rng = np.random.default_rng(17)
+    pts, k = [], 0
+    for rep in range(6):
+        for size in sizes:
+            at = np.array([k % 8, (k // 8) % 8, 0.0])[:dim] * 12 * dx
+            # well separated points of a cluster: a jittered corner of the lattice
+            g = np.array([[i, j, m][:dim] for m in range(3) for j in range(3) for i in range(2)], dtype=float)
+            g = np.unique(g, axis=0)
+            g = g[rng.permutation(len(g))[:min(size, len(g))]]
+            pts.append(at + dx * (g + rng.uniform(-0.1, 0.1, g.shape)))
+            k += 1
+    x = np.concatenate(pts)
+    n = len(x)
+    c.x = np.ascontiguousarray(x)
+    c.v = rng.uniform(-0.1, 0.1, x.shape)
+    c.rho = s.rho_rest * (1.0 + rng.uniform(-5e-3, 5e-3, n))
+    b = s.rho_rest * s.speed_sound ** 2 / s.gam
+    c.p = b * ((c.rho / s.rho_rest) ** s.gam - 1.0)
+    c.m = np.full(n, s.rho_rest * dx ** dim)
+    c.b = np.full(n, abi.FREE, dtype=np.int32)
+    c.n_bound = 0
+    c.blocks = [dict(first=0, last=n, is_fluid=1)]
+    return c
+
+
+@pytest.mark.parametrize("precision", [abi.PREC_FP64, abi.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("dim,ale,sizes", [(2, 0, SIZES), (3, 0, SIZES), (3, 1, SIZES), (3, 0, (1,))],
+                         ids=["2d", "3d", "3d-ale", "3d-lone"])
+def test_row_remainders(dim, ale, sizes, precision):
+    case = _clusters(dim, sizes, precision, ale)
+    print(f"[walk] {dim}D ale={ale} sizes={sizes} n={case.n} precision={precision}", flush=True)
+    eng, orc = _engine(case), _oracle(case)
+    eng.build_neighbours()
+    orc.build_neighbours()
+    off_e, idx_e = eng.neighbours()
+    off_o, idx_o, _ = orc.neighbours()
+    assert same_neighbour_sets(off_e, idx_e, off_o, idx_o)
+    tol = FP64_PASS if precision == abi.PREC_FP64 else MIXED_STEP
+    npd_e, npd_o = eng.dsph_prestep(), orc.dsph_prestep()
+    assert abs(npd_e - npd_o) <= tol * abs(npd_o)
+    # sums that do not pass through the correction matrix, whose inverse is
+    # ill-conditioned for a handful of neighbours
+    for f in ("KERNSUM", "COLOUR"):
+        assert_close(f, eng.field(f), orc.field(f), tol)
+    eng.detect_surface()
+    orc.detect_surface()
+    assert np.array_equal(eng.field("SURF"), orc.field("SURF"))
+    eng.dissipation_terms()
+    orc.dissipation_terms()
+    assert_close("AVISC", eng.field("AVISC"), orc.field("AVISC"), tol)
+    if sizes == (1,):
+        npd_o = 1.0 / case.settings.particle_step ** dim  # no pair gives it
+    eng.acc_rrho(npd_o)
+    orc.acc_rrho(npd_o)
+    assert_close("ACC", eng.field("ACC"), orc.field("ACC"), tol)
+    eng.close()
