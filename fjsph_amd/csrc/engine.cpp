@@ -664,6 +664,22 @@ void group_blocks(fjsph_ctx* ctx)
                           ctx->st));
 }
 
+/* Targets per tile block where the caller has set none.  A block of 256
+ * stages a candidate for the fewest targets' worth of work and is the
+ * fastest for large sets; below about a million particles it leaves too few
+ * blocks for 256 CUs, and blocks of 128 and 64, whose waves share the lists
+ * (Split), win although they stage more.  ms a step with 256 / 128 / 64
+ * targets, 3D: 100k Runge-Kutta 4.39 / 3.22 / 3.11, 200k FP64 12.7 / 10.6 /
+ * 10.3, 268k 13.4 / 11.5 / 11.6, 700k 9.17 / 8.96 / 10.75, 1M 14.5 / 14.5 /
+ * 17.7.  In 2D a target has a tenth of the neighbours, so blocks are shorter
+ * work and the lines lie lower: 6.5k 1.29 / 1.22 / 1.18, 23k 1.34 / 1.11 /
+ * 1.20, 86k 1.51 / 1.31 / 1.48, 345k 2.39 / 2.30 / 2.88. */
+int32_t default_targets(int dim, int64_t n)
+{
+    const int64_t n64 = dim == 3 ? 250000 : 15000, n128 = dim == 3 ? 1000000 : 500000;
+    return n < n64 ? 64 : n < n128 ? 128 : 256;
+}
+
 void build_neighbours(fjsph_ctx* ctx, bool reorder)
 {
     PassTimer t(ctx, FJSPH_T_NEIGHBOUR);
@@ -743,7 +759,7 @@ void build_neighbours(fjsph_ctx* ctx, bool reorder)
     int32_t C;
     {
         const double occ = std::pow(cs / ctx->s.particle_step, D);
-        const double targets = ctx->block_targets > 0 ? double(ctx->block_targets) : 256.0;
+        const double targets = ctx->block_targets > 0 ? double(ctx->block_targets) : double(default_targets(D, n));
         C = int32_t(std::lround(targets / std::max(occ, 1.0)));
         /* at most kMaxBlockCells cells per block: the list build's FP32
          * prefilter band (k_build_t) holds for blocks up to that length */

@@ -66,10 +66,11 @@ struct NbrList {
 constexpr int TILE = FJ_TILE;
 static_assert(TILE % 4 == 0, "tile slots come in groups of 4");
 constexpr uint32_t NO_ENTRY = 0xFFFF;
-/* Room past the list rows: the walks load one row past a wave's last one,
- * and the lanes past a block's targets load the positions after them (what
- * they read is masked by the targets' row counts). */
-constexpr int kRowSlack = 1;
+/* Room past the list rows: the up to four waves that share a list load one
+ * row each past its last one, and the lanes past a block's targets load the
+ * positions after them (what they read is masked by the targets' row
+ * counts). */
+constexpr int kRowSlack = 4;
 constexpr int kTargetSlack = 256;
 /* Longest tile block in cells: every coordinate of a block's candidate
  * union then lies within 1000 H of its first target, the bound the FP32

@@ -191,6 +191,58 @@ __device__ __forceinline__ void split_rel(double x, double ref, float& hi, float
     lo = float(d - double(hi));
 }
 
+/* How the waves of a block share its targets.  A block with more than two
+ * waves' worth of targets gives each wave 64 of them; in a block with fewer
+ * the waves left over take part in the same lists: `n` waves walk every
+ * n-th row of the same 64 targets and their sums meet at the end
+ * (split_fold).  A particle set that gives each CU less than a few blocks
+ * runs on short blocks (build_neighbours) and so on four waves a list. */
+struct Split {
+    int n, part, lane; /* waves to a list, this wave's place among them, the thread's target */
+};
+
+__device__ __forceinline__ Split split_of(const BlockHead& h)
+{
+    const int nw = __builtin_amdgcn_readfirstlane((h.p1 - h.p0 + 63) >> 6);
+    const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    Split s;
+    s.n = nw <= 1 ? NWAVE : nw == 2 ? NWAVE / 2 : 1;
+    const int tw = NWAVE / s.n; /* waves with targets of their own */
+    s.part = w / tw;
+    s.lane = int(threadIdx.x) - s.part * tw * 64;
+    return s;
+}
+
+/* Values of the waves of a list folded in wave order into the first one's;
+ * `buf` is LDS of 3 TPB values that the block is done with. */
+template <int N, typename Op>
+__device__ __forceinline__ void split_fold(const Split& sp, double (&v)[N], double* buf, Op op)
+{
+    if (sp.n == 1) return;
+#pragma unroll
+    for (int r = 0; r < N; r += 3) {
+        __syncthreads();
+#pragma unroll
+        for (int k = r; k < (r + 3 < N ? r + 3 : N); ++k) buf[(k - r) * TPB + threadIdx.x] = v[k];
+        __syncthreads();
+        if (sp.part == 0) {
+            const int step = TPB / sp.n;
+#pragma unroll
+            for (int k = r; k < (r + 3 < N ? r + 3 : N); ++k)
+                for (int q = 1; q < sp.n; ++q) v[k] = op(v[k], buf[(k - r) * TPB + threadIdx.x + q * step]);
+        }
+    }
+}
+static_assert(sizeof(float4) * TILE >= 3 * sizeof(double) * TPB, "a tile array serves as split_fold's buffer");
+
+template <typename Op>
+__device__ __forceinline__ double split_fold1(const Split& sp, double v, double* buf, Op op)
+{
+    double a[1] = {v};
+    split_fold(sp, a, buf, op);
+    return a[0];
+}
+
 /* ------------------------------------------------------------ list rows */
 
 /* Lock-step walk of one target's rows: `row` advances in every lane of the
@@ -206,21 +258,24 @@ __device__ __forceinline__ void split_rel(double x, double ref, float& hi, float
  * lane has an entry of it left, so a lane that dropped out could leave the
  * others on padding rows of the tile. */
 struct Rows {
-    const uint64_t* rp; /* the next row, at position 0 */
+    const uint64_t* rp; /* the wave's next row, at position 0 */
     int64_t stride;
     uint32_t p;
     int row, nrows;
     bool on;
     uint64_t u;
-    __device__ __forceinline__ void init(const NbrList& nl, int p_, int nrows_, bool on_)
+    int step;
+    __device__ __forceinline__ void init(const NbrList& nl, int p_, int nrows_, bool on_, const Split& sp)
     {
         on = on_;
         nrows = nrows_;
-        stride = nl.npad;
+        step = sp.n;
+        stride = sp.n * nl.npad;
         p = uint32_t(p_);
-        row = 0;
-        u = nl.lu4[p];
-        rp = nl.lu4 + stride;
+        row = sp.part;
+        const uint64_t* first = nl.lu4 + sp.part * nl.npad;
+        u = first[p];
+        rp = first + stride;
     }
     /* the current row is one of the lane's and lies in the tile that ends
      * below `top` */
@@ -230,7 +285,7 @@ struct Rows {
         const uint64_t cur = u;
         u = rp[p];
         rp += stride;
-        ++row;
+        row += step;
         return cur;
     }
 };
@@ -660,6 +715,22 @@ __device__ __forceinline__ double dsph_pair(const Consts& c, double inv_H, const
     return W;
 }
 
+/* The pair sums of the waves that share a list, together. */
+template <int D>
+__device__ __forceinline__ void dsph_fold(const Split& sp, double* buf, double (&Lm)[D * (D + 1) / 2],
+                                          double (&Lnb)[D * (D + 1) / 2], double (&gR)[D], double (&nr)[D],
+                                          double& kernsum, double& colour)
+{
+    split_fold(sp, Lm, buf, OpSum());
+    split_fold(sp, Lnb, buf, OpSum());
+    split_fold(sp, gR, buf, OpSum());
+    split_fold(sp, nr, buf, OpSum());
+    double kc[2] = {kernsum, colour};
+    split_fold(sp, kc, buf, OpSum());
+    kernsum = kc[0];
+    colour = kc[1];
+}
+
 /* Per-slot outputs of the dSPH_PreStep pair sums. */
 template <int D>
 __device__ __forceinline__ void dsph_out(DevState& s, Aux& ax, int64_t i, const double (&Lm)[D * (D + 1) / 2],
@@ -705,8 +776,9 @@ __global__ __launch_bounds__(TPB) void k_dsph_t(Consts c, DevState s, Aux ax, Ti
     const int NT = n_tiles(U);
     double npd_acc = 0.0;
     const double inv_H = 1.0 / c.H;
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         double xi[D], xbi[D], Lm[NS], Lnb[NS], gR[D], nr[D];
@@ -720,9 +792,9 @@ __global__ __launch_bounds__(TPB) void k_dsph_t(Consts c, DevState s, Aux ax, Ti
 #pragma unroll
         for (int k = 0; k < NS; ++k) { Lm[k] = 0.0; Lnb[k] = 0.0; }
         const double rhoi = active ? s.rho[i] : 0.0;
-        double kernsum = c.Wc, colour = 0.0;
+        double kernsum = sp.part == 0 ? c.Wc : 0.0, colour = 0.0;
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, active);
+        cu.init(nl, p, active ? nl.count[i] : 0, active, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -749,7 +821,8 @@ __global__ __launch_bounds__(TPB) void k_dsph_t(Consts c, DevState s, Aux ax, Ti
                                         kernsum, colour);
             FJ_TILE_ENTRIES_END(cu, nl)
         }
-        if (active) dsph_out<D>(s, ax, i, Lm, Lnb, gR, nr, kernsum, colour);
+        dsph_fold<D>(sp, &tp[0][0], Lm, Lnb, gR, nr, kernsum, colour);
+        if (active && sp.part == 0) dsph_out<D>(s, ax, i, Lm, Lnb, gR, nr, kernsum, colour);
     }
     const double bs = block_reduce(npd_acc, OpSum(), lds);
     if (threadIdx.x == 0) partial[h.b] = bs;
@@ -790,8 +863,9 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
     const float Ht = float(c.H), inv_Hf = float(1.0 / c.H), Wcf = float(c.Wc);
     const double inv_H = 1.0 / c.H;
     double npd_acc = 0.0;
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool slow = active && nl.nnb[i] < 2 * D;
@@ -804,14 +878,14 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
         const double rhoi = active ? s.rho[i] : rref;
         float drhoi, rlo;
         split_rel(rhoi, rref, drhoi, rlo);
-        double Lm[NS], Lnb[NS], gR[D], nr[D], kernsum = c.Wc, colour = 0.0;
+        double Lm[NS], Lnb[NS], gR[D], nr[D], kernsum = sp.part == 0 ? c.Wc : 0.0, colour = 0.0;
         float fLm[NS], fLnb[NS], fgR[D], fnr[D], fks = 0.f, fcol = 0.f;
 #pragma unroll
         for (int k = 0; k < NS; ++k) { Lm[k] = 0.0; Lnb[k] = 0.0; fLm[k] = 0.f; fLnb[k] = 0.f; }
 #pragma unroll
         for (int a = 0; a < D; ++a) { gR[a] = 0.0; nr[a] = 0.0; fgR[a] = 0.f; fnr[a] = 0.f; }
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, active && !slow);
+        cu.init(nl, p, active ? nl.count[i] : 0, active && !slow, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -912,7 +986,7 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
             fks = 0.f;
             fcol = 0.f;
         }
-        if (slow) {
+        if (slow && sp.part == 0) {
             double xi[D], xbi[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) {
@@ -935,7 +1009,8 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
                 }
             }
         }
-        if (active) dsph_out<D>(s, ax, i, Lm, Lnb, gR, nr, kernsum, colour);
+        dsph_fold<D>(sp, reinterpret_cast<double*>(tA), Lm, Lnb, gR, nr, kernsum, colour);
+        if (active && sp.part == 0) dsph_out<D>(s, ax, i, Lm, Lnb, gR, nr, kernsum, colour);
     }
     const double bs = block_reduce(npd_acc, OpSum(), lds);
     if (threadIdx.x == 0) partial[h.b] = bs;
@@ -1195,8 +1270,9 @@ __global__ __launch_bounds__(TPB) void k_surface1_t(Consts c, DevState s, Aux ax
     const double inv_H = 1.0 / c.H;
     const double h133 = 1.33 * c.particle_step;
     const double r_lim = sqrt(2.0) * h133;
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
@@ -1233,7 +1309,7 @@ __global__ __launch_bounds__(TPB) void k_surface1_t(Consts c, DevState s, Aux ax
         const T Bg = T(c.B * c.gam), cfac = T(sqrt(c.B * c.gam / rhoi)), Ht = T(c.H);
         const T eps2 = T(0.0001 * c.H_sq), alpha = T(c.visc_alpha);
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, fluid);
+        cu.init(nl, p, active ? nl.count[i] : 0, fluid, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -1316,7 +1392,15 @@ __global__ __launch_bounds__(TPB) void k_surface1_t(Consts c, DevState s, Aux ax
                 }
             FJ_TILE_ENTRIES_END(cu, nl)
         }
-        if (active) surface1_out<D, MODE>(c, s, i, fluid, bi, lam_nb, lami, found, nrm, av, rd, norms_tmp, ax.nhat);
+        if constexpr (with_surf) {
+            split_fold(sp, nrm, &tp[0][0], OpSum());
+            found = split_fold1(sp, found ? 1.0 : 0.0, &tp[0][0], OpMax()) != 0.0;
+        }
+        if constexpr (with_diss) {
+            split_fold(sp, av, &tp[0][0], OpSum());
+            rd = split_fold1(sp, rd, &tp[0][0], OpSum());
+        }
+        if (active && sp.part == 0) surface1_out<D, MODE>(c, s, i, fluid, bi, lam_nb, lami, found, nrm, av, rd, norms_tmp, ax.nhat);
     }
 }
 
@@ -1371,8 +1455,9 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
     const float Ht = float(c.H), inv_H = float(1.0 / c.H), Wc = float(c.Wc);
     const float eps2 = float(0.0001 * c.H_sq), alpha = float(c.visc_alpha);
     const float rreff = float(rref);
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
@@ -1427,7 +1512,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
         const float rhoif = float(rhoi);
         const float cfac = float(sqrt(c.B * c.gam / rhoi));
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, fluid);
+        cu.init(nl, p, active ? nl.count[i] : 0, fluid, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -1534,7 +1619,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
                         if (sure) found = q > 0.f;
                         else {
                             /* rare: the slot goes straight to memory */
-                            if (npend < kSurfPendMax)
+                            if (npend < kSurfPendMax && sp.n == 1)
                                 reinterpret_cast<int32_t*>(ax.spend)[i * kSurfPendMax + npend] = tsl[with_surf ? t[e] : 0];
                             ++npend;
                         }
@@ -1588,6 +1673,21 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
             rd += double(frd);
             frd = 0.f;
         }
+        double* const buf = reinterpret_cast<double*>(tA);
+        if constexpr (with_surf) {
+            split_fold(sp, nrm, buf, OpSum());
+            /* waves that share a list keep no slots of their undecided
+             * pairs: k_surface1_resolve then goes through the list */
+            double fp[2] = {found ? 1.0 : 0.0, double(npend > 0 && sp.n > 1 ? kSurfPendMax + 1 : npend)};
+            split_fold(sp, fp, buf, OpMax());
+            found = fp[0] != 0.0;
+            npend = int(fp[1]);
+        }
+        if constexpr (with_diss) {
+            split_fold(sp, av, buf, OpSum());
+            rd = split_fold1(sp, rd, buf, OpSum());
+        }
+        if (sp.part != 0) continue;
         if (active) surface1_out<D, MODE>(c, s, i, fluid, bi, lam_nb, lami, found, nrm, av, rd, norms_tmp, ax.nhat);
         if constexpr (with_surf) {
             /* undecided: k_surface1_resolve sets the flag from the FP64 test */
@@ -1705,8 +1805,9 @@ __global__ __launch_bounds__(TPB) void k_surface2_t(Consts c, DevState s, Aux ax
     const int U = h.pre[h.nseg];
     const int NT = n_tiles(U);
     const double inv_H = 1.0 / c.H;
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
@@ -1732,7 +1833,7 @@ __global__ __launch_bounds__(TPB) void k_surface2_t(Consts c, DevState s, Aux ax
         double curve = 0.0, qmax = 0.0;
         int zone = (fluid && s.surf[i] == 1) ? 1 : 0;
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, fluid);
+        cu.init(nl, p, active ? nl.count[i] : 0, fluid, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -1779,7 +1880,12 @@ __global__ __launch_bounds__(TPB) void k_surface2_t(Consts c, DevState s, Aux ax
                 if (tsurf[t] == 1) zone = 1;
             FJ_TILE_ENTRIES_END(cu, nl)
         }
-        if (!fluid) continue;
+        curve = split_fold1(sp, curve, &tp[0][0], OpSum());
+        double qz[2] = {qmax, double(zone)};
+        split_fold(sp, qz, &tp[0][0], OpMax());
+        qmax = qz[0];
+        zone = int(qz[1]);
+        if (!fluid || sp.part != 0) continue;
         const double wo = (occl && Vdn > 0.0) ? qmax / Vdn : 0.0;
         s.woccl[i] = s.lam_nb[i] < c.lam_cutoff ? fmax(0.0, fmin(wo, 1.0)) : 1.0;
         double nh[D];
@@ -1825,8 +1931,9 @@ __global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevSt
         }
     }
     const float Ht = float(c.H), inv_Hf = float(1.0 / c.H), Wcf = float(c.Wc);
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
@@ -1859,7 +1966,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevSt
         float fcurve = 0.f, qmax = 0.f;
         bool zone = fluid && s.surf[i] == 1;
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, fluid);
+        cu.init(nl, p, active ? nl.count[i] : 0, fluid, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -1940,7 +2047,13 @@ __global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevSt
             curve += double(fcurve);
             fcurve = 0.f;
         }
-        if (!fluid) continue;
+        double* const buf = reinterpret_cast<double*>(tA);
+        curve = split_fold1(sp, curve, buf, OpSum());
+        double qz[2] = {double(qmax), zone ? 1.0 : 0.0};
+        split_fold(sp, qz, buf, OpMax());
+        qmax = float(qz[0]);
+        zone = qz[1] != 0.0;
+        if (!fluid || sp.part != 0) continue;
         const double Vdn = sqrt(dotd<D>(Vd64, Vd64));
         const double wo = (occl && Vdn > 0.0) ? double(qmax) / Vdn : 0.0;
         s.woccl[i] = s.lam_nb[i] < c.lam_cutoff ? fmax(0.0, fmin(wo, 1.0)) : 1.0;
@@ -2044,8 +2157,9 @@ __global__ __launch_bounds__(TPB) void k_shift_t(Consts c, DevState s, Aux ax, c
     const int NT = n_tiles(U);
     const double inv_H = 1.0 / c.H;
     const double inv_Wdx = 1.0 / c.W_dx;
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
@@ -2062,7 +2176,7 @@ __global__ __launch_bounds__(TPB) void k_shift_t(Consts c, DevState s, Aux ax, c
         }
         double maxU2 = 0.0, dmin = 2.0;
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, work);
+        cu.init(nl, p, active ? nl.count[i] : 0, work, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -2109,7 +2223,10 @@ __global__ __launch_bounds__(TPB) void k_shift_t(Consts c, DevState s, Aux ax, c
                 if (dv2 > maxU2) maxU2 = dv2;
             FJ_TILE_ENTRIES_END(cu, nl)
         }
-        if (fluid) shift_out<D>(c, s, i, work, lam_nb, vi, nhat, du, maxU2, dmin, s.surfzone[i]);
+        split_fold(sp, du, &tp[0][0], OpSum());
+        maxU2 = split_fold1(sp, maxU2, &tp[0][0], OpMax());
+        dmin = split_fold1(sp, dmin, &tp[0][0], OpMin());
+        if (fluid && sp.part == 0) shift_out<D>(c, s, i, work, lam_nb, vi, nhat, du, maxU2, dmin, s.surfzone[i]);
     }
 }
 
@@ -2144,8 +2261,9 @@ __global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState
         }
     }
     const float Ht = float(c.H), inv_Hf = float(1.0 / c.H), Wcf = float(c.Wc), inv_Wdx = float(1.0 / c.W_dx);
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
@@ -2165,7 +2283,7 @@ __global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState
         float maxU2 = 0.f;
         double dmin = 2.0;
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, work);
+        cu.init(nl, p, active ? nl.count[i] : 0, work, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -2246,7 +2364,11 @@ __global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState
                 fdu[a] = 0.f;
             }
         }
-        if (!fluid) continue;
+        double* const buf = reinterpret_cast<double*>(tA);
+        split_fold(sp, du, buf, OpSum());
+        maxU2 = float(split_fold1(sp, double(maxU2), buf, OpMax()));
+        dmin = split_fold1(sp, dmin, buf, OpMin());
+        if (!fluid || sp.part != 0) continue;
         double vi[D];
 #pragma unroll
         for (int a = 0; a < D; ++a) vi[a] = work ? s.v[i * D + a] : 0.0;
@@ -2325,8 +2447,9 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
      * is 1e-5 */
     const double cos15 = cos(kPi / 12.0);
     const float ang_yes_lo = float(-1.0 + 1e-5), ang_yes_hi = float(cos15 - 1e-5), ang_no = float(cos15 + 1e-5);
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
@@ -2367,7 +2490,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
         float fcurve = 0.f, qmax = 0.f, maxU2 = 0.f;
         bool zone = fluid && s.surf[i] == 1, wide = false;
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, fluid);
+        cu.init(nl, p, active ? nl.count[i] : 0, fluid, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -2495,7 +2618,16 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
                 fdu[a] = 0.f;
             }
         }
-        if (!fluid) continue;
+        double* const buf = reinterpret_cast<double*>(tA);
+        split_fold(sp, du, buf, OpSum());
+        curve = split_fold1(sp, curve, buf, OpSum());
+        double mx[4] = {double(qmax), double(maxU2), zone ? 1.0 : 0.0, wide ? 1.0 : 0.0};
+        split_fold(sp, mx, buf, OpMax());
+        qmax = float(mx[0]);
+        maxU2 = float(mx[1]);
+        zone = mx[2] != 0.0;
+        wide = mx[3] != 0.0;
+        if (!fluid || sp.part != 0) continue;
         double Vd64[D];
 #pragma unroll
         for (int a = 0; a < D; ++a)
@@ -2928,8 +3060,9 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_t(Consts c, DevState
     const double eps2 = 0.001 * c.H_sq;
     const double nu = c.nu;
     const double contang_fac = 1.0 + 0.5 * cos(0.5 * kPi * 7.0 / 9.0);
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
@@ -2953,7 +3086,7 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_t(Consts c, DevState
         for (int a = 0; a < D; ++a) acc[a] = 0.0;
         double Rrho_ = 0.0, Rrhoc_ = 0.0;
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, fluid);
+        cu.init(nl, p, active ? nl.count[i] : 0, fluid, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -3041,7 +3174,12 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_t(Consts c, DevState
                 }
             FJ_TILE_ENTRIES_END(cu, nl)
         }
-        if (!fluid) continue;
+        split_fold(sp, acc, &ft.P[0][0], OpSum());
+        double rr2[2] = {Rrho_, Rrhoc_};
+        split_fold(sp, rr2, &ft.P[0][0], OpSum());
+        Rrho_ = rr2[0];
+        Rrhoc_ = rr2[1];
+        if (!fluid || sp.part != 0) continue;
 #pragma unroll
         for (int a = 0; a < D; ++a) s.acc[i * D + a] = acc[a];
         s.Rrho[i] = c.ale ? (Rrho_ * rhoi + Rrhoc_ + s.deltaD[i]) : (Rrho_ * rhoi + s.deltaD[i]);
@@ -3110,8 +3248,9 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
     const float eps2 = float(0.001 * c.H_sq);
     const float nu = float(c.nu);
     const float contang_fac = float(1.0 + 0.5 * cos(0.5 * kPi * 7.0 / 9.0));
+    const Split sp = split_of(h);
     for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
+        const int p = pb + sp.lane;
         const bool active = p < h.p1;
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
@@ -3138,7 +3277,7 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
         for (int a = 0; a < D; ++a) acc[a] = 0.0;
         double Rrho_ = 0.0, Rrhoc_ = 0.0, vS = 0.0;
         Rows cu;
-        cu.init(nl, p, active ? nl.count[i] : 0, fluid);
+        cu.init(nl, p, active ? nl.count[i] : 0, fluid, sp);
         TileSlots ts;
         ts.load(tg, h, 0, NT, U);
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
@@ -3275,7 +3414,14 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
                 vS += double(vs);
             }
         }
-        if (!fluid) continue;
+        double* const buf = reinterpret_cast<double*>(ft.A);
+        split_fold(sp, acc, buf, OpSum());
+        double rr3[3] = {Rrho_, Rrhoc_, vS};
+        split_fold(sp, rr3, buf, OpSum());
+        Rrho_ = rr3[0];
+        Rrhoc_ = rr3[1];
+        vS = rr3[2];
+        if (!fluid || sp.part != 0) continue;
         if constexpr (ALE) {
 #pragma unroll
             for (int a = 0; a < D; ++a) acc[a] += 2.0 * s.v[i * D + a] * vS;

@@ -2,13 +2,14 @@
 that every target has k - 1 neighbours (no row at all, rows of one to four
 entries, a second row with one) and the waves mix lanes with and without
 entries.  Pair sums against the oracle; FP64 to summation order, mixed to the
-FP32 pair terms (as test_gpu_parity.py)."""
+FP32 pair terms (as test_gpu_parity.py).  And blocks short enough that two or
+four waves share a target's list."""
 import numpy as np
 import pytest
 
 from fjsph_amd import abi, cases
 from tests.parity import assert_close, same_neighbour_sets
-from tests.test_gpu_parity import FP64_PASS, MIXED_STEP, _engine, _oracle
+from tests.test_gpu_parity import FP64_PASS, FP64_STEP, MIXED_STEP, _engine, _oracle, _small_cases
 
 pytestmark = pytest.mark.gpu
 
@@ -75,4 +76,28 @@ def test_row_remainders(dim, ale, sizes, precision):
     eng.acc_rrho(npd_o)
     orc.acc_rrho(npd_o)
     assert_close("ACC", eng.field("ACC"), orc.field("ACC"), tol)
+    eng.close()
+
+
+@pytest.mark.parametrize("precision", [abi.PREC_FP64, abi.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("targets", [16, 64, 128, 192])
+@pytest.mark.parametrize("name", ["dam2d", "jet3d_ale", "drop3d"])
+def test_shared_lists(name, targets, precision):
+    """Start-up pass and two steps with blocks of few targets: four waves to
+    a list (16, 64), two (128), one (192), and a run's mixture of them."""
+    case = dict(_small_cases())[name]
+    case.settings.precision = precision
+    print(f"[walk] {name}: n={case.n} {targets} targets a block, precision={precision}", flush=True)
+    eng, orc = _engine(case), _oracle(case)
+    eng.set_block_targets(targets)
+    eng.integrate_no_update()
+    orc.integrate_no_update()
+    for _ in range(2):
+        ie, io = eng.integrate_step(), orc.integrate_step()
+        if precision == abi.PREC_FP64:
+            assert ie["iterations"] == io["iterations"]
+    tol = FP64_STEP if precision == abi.PREC_FP64 else MIXED_STEP
+    assert np.array_equal(eng.field("SURF"), orc.field("SURF"))
+    for f in ("X", "V", "RHO", "ACC", "RRHO", "LAM", "AVISC"):
+        assert_close(f, eng.field(f), orc.field(f), tol)
     eng.close()
