@@ -653,7 +653,8 @@ double group_layout(fjsph_ctx* ctx, double cs)
 void group_blocks(fjsph_ctx* ctx)
 {
     const int D = ctx->s.dim, G = ctx->ngroups;
-    const int64_t per_layer = (D == 3 ? int64_t(ctx->tg.dims[1]) : 1) * ctx->tg.nchunk;
+    /* blocks of grouped contexts are one layer thick along the last axis */
+    const int64_t per_layer = (D == 3 ? int64_t(ctx->tg.nb[1]) : 1) * ctx->tg.nb[0];
     ctx->gblk_h.assign(size_t(G) + 1, 0);
     for (int g = 0; g < G; ++g) ctx->gblk_h[g] = int64_t(ctx->gl0_h[g * 2]) * per_layer;
     ctx->gblk_h[G] = int64_t(ctx->gl0_h[(G - 1) * 2] + ctx->gl0_h[(G - 1) * 2 + 1]) * per_layer;
@@ -666,18 +667,56 @@ void group_blocks(fjsph_ctx* ctx)
 
 /* Targets per tile block where the caller has set none.  A block of 256
  * stages a candidate for the fewest targets' worth of work and is the
- * fastest for large sets; below about a million particles it leaves too few
- * blocks for 256 CUs, and blocks of 128 and 64, whose waves share the lists
- * (Split), win although they stage more.  ms a step with 256 / 128 / 64
- * targets, 3D: 100k Runge-Kutta 4.39 / 3.22 / 3.11, 200k FP64 12.7 / 10.6 /
- * 10.3, 268k 13.4 / 11.5 / 11.6, 700k 9.17 / 8.96 / 10.75, 1M 14.5 / 14.5 /
- * 17.7.  In 2D a target has a tenth of the neighbours, so blocks are shorter
- * work and the lines lie lower: 6.5k 1.29 / 1.22 / 1.18, 23k 1.34 / 1.11 /
- * 1.20, 86k 1.51 / 1.31 / 1.48, 345k 2.39 / 2.30 / 2.88. */
-int32_t default_targets(int dim, int64_t n)
+ * fastest for large sets; below a few hundred thousand particles it leaves
+ * too few blocks for 256 CUs, and blocks of 128 and 64, whose waves share
+ * the lists (Split), win although they stage more.  ms a step with 256 / 128
+ * / 64 targets, 3D: 100k Runge-Kutta 4.14 / 3.18 / 3.09, 268k 12.9 / 11.5 /
+ * 11.4, 700k 9.00 / 8.98 / 10.9, 1M 14.4 / 14.7 / 18.2.  In 2D a target has a tenth of the neighbours, so blocks are
+ * shorter work and the line lies lower: 6.5k 1.24 / 1.13 / 1.16, 86k 1.39 /
+ * 1.41 / 1.56, 345k 2.04 / 2.39 / 2.99.  FP64 keeps its blocks, see
+ * block_shape. */
+int32_t default_targets(int dim, int64_t n, bool f32)
 {
-    const int64_t n64 = dim == 3 ? 250000 : 15000, n128 = dim == 3 ? 1000000 : 500000;
-    return n < n64 ? 64 : n < n128 ? 128 : 256;
+    if (!f32) return 256;
+    if (dim == 2) return n < 60000 ? 128 : 256;
+    return n < 250000 ? 64 : n < 700000 ? 128 : 256;
+}
+
+/* Cells of a tile block along each axis for about `cells` cells.  Compact
+ * boxes have the smallest candidate unions: the 4 cells of a block of 256
+ * targets in a row need 54 cells' candidates staged, as two rows of two they
+ * need 48, and of a 2D block of 38 cells 120 or, as 6 x 6, 64 (345k
+ * particles: 2.39 -> 2.04 ms a step; 1M jet 14.5 -> 14.3, 1M jet in
+ * crossflow 21.5 -> 20.7, 256 drops 30.7 -> 29.4).  The rows of the union keep to kMaxRows, so a
+ * long block grows along x, up to kMaxBlockCells cells (the list build's
+ * FP32 prefilter band holds up to that length).  Independent simulations
+ * are stacked along the last axis one empty layer apart, so that their
+ * blocks stay one layer thick.  In FP64 the blocks are rows of cells for
+ * about 256 targets whatever the particle count: the order of every sum
+ * follows the blocks, a droplet's sub-iterations end on changes at the
+ * rounding level of its positions, and with another order a 1.4 mm droplet's
+ * pressures moved by 2.2e-10 over 20 steps, more than an FP64 run is held
+ * to. */
+void block_shape(int dim, bool one_layer, bool f32, double cells, const int32_t (&dims)[3], int32_t (&bc)[3])
+{
+    const int across = !f32 ? 0 : dim - 1 - (one_layer ? 1 : 0); /* axes other than x to grow along */
+    bc[0] = bc[1] = bc[2] = 1;
+    if (across > 0) {
+        const int32_t most = dim == 3 && across == 2 ? 3 : dim == 3 ? 6 : kMaxRows - 2;
+        /* the largest edge whose box has at most about `cells` cells */
+        for (int32_t e = 2; e <= most; ++e)
+            if (std::pow(double(e), across + 1) <= 1.05 * cells) bc[1] = e;
+        bc[1] = std::min(bc[1], dims[1]);
+        if (across == 2) bc[2] = std::min(bc[1], dims[2]);
+    }
+    const double per = double(bc[1]) * bc[2];
+    bc[0] = int32_t(std::max(1.0, std::floor(cells / per + 0.5)));
+    if (across == 2 && bc[1] == 1 && bc[0] >= 4) {
+        /* 4 to 7 cells: two rows of half as many */
+        bc[1] = std::min(2, dims[1]);
+        bc[0] = bc[0] / bc[1];
+    }
+    bc[0] = std::max(1, std::min({bc[0], dims[0], kMaxBlockCells}));
 }
 
 void build_neighbours(fjsph_ctx* ctx, bool reorder)
@@ -735,18 +774,22 @@ void build_neighbours(fjsph_ctx* ctx, bool reorder)
         if (ctx->ncols > 0) launch_inlet_backslot(ctx->col, ctx->depth, n, ctx->c_back, ctx->st);
     }
     HIPCHK(hipMemcpyAsync(ctx->aux.xb, ctx->pnp1.x, sizeof(double) * n * D, hipMemcpyDeviceToDevice, ctx->st));
-    /* tile grid: chunks of C cells sized for about one workgroup of targets */
-    auto set_tiles = [&](int32_t C) {
+    /* tile grid: boxes of cells sized for the block's targets */
+    auto set_tiles = [&](const int32_t (&bc)[3]) {
         TileGrid& tg = ctx->tg;
-        for (int k = 0; k < 3; ++k) tg.dims[k] = ctx->dims[k];
-        tg.C = C;
-        tg.nchunk = (ctx->dims[0] + C - 1) / C;
-        tg.nblocks = int64_t(ctx->dims[1]) * ctx->dims[2] * tg.nchunk;
+        tg.nblocks = 1;
+        for (int k = 0; k < 3; ++k) {
+            tg.dims[k] = ctx->dims[k];
+            tg.bc[k] = bc[k];
+            tg.nb[k] = (ctx->dims[k] + bc[k] - 1) / bc[k];
+            tg.nblocks *= tg.nb[k];
+        }
         tg.start = ctx->cell_start;
         tg.order = ctx->order;
         tg.vorder = ctx->vorder;
         tg.pos = ctx->pos;
         tg.cell = ctx->cell;
+        tg.share = ctx->nl.f32;
         tg.lgrp = grouped(ctx) ? ctx->lgrp : nullptr;
         tg.gactive = grouped(ctx) ? ctx->gactive : nullptr;
         tg.gnpd = grouped(ctx) ? ctx->gnpd : nullptr;
@@ -756,16 +799,14 @@ void build_neighbours(fjsph_ctx* ctx, bool reorder)
             dalloc(ctx->partial, size_t(std::max<int64_t>(ctx->partial_cap, int64_t(ctx->nparts) * 8)));
         }
     };
-    int32_t C;
+    int32_t bc[3];
     {
         const double occ = std::pow(cs / ctx->s.particle_step, D);
-        const double targets = ctx->block_targets > 0 ? double(ctx->block_targets) : double(default_targets(D, n));
-        C = int32_t(std::lround(targets / std::max(occ, 1.0)));
-        /* at most kMaxBlockCells cells per block: the list build's FP32
-         * prefilter band (k_build_t) holds for blocks up to that length */
-        C = std::max(1, std::min({C, ctx->dims[0], kMaxBlockCells}));
+        const double targets =
+            ctx->block_targets > 0 ? double(ctx->block_targets) : double(default_targets(D, n, ctx->nl.f32 != 0));
+        block_shape(D, grouped(ctx), ctx->nl.f32 != 0, std::max(1.0, targets / std::max(occ, 1.0)), ctx->dims, bc);
     }
-    set_tiles(C);
+    set_tiles(bc);
     for (int attempt = 0; attempt < 40; ++attempt) {
         HIPCHK(hipMemsetAsync(&ctx->sc->max_count, 0, 2 * sizeof(int32_t), ctx->st));
         launch_build_lists(D, ctx->pnp1.x, n, ctx->tg, ctx->d.sr, ctx->nl, ctx->sc, ctx->st);
@@ -774,8 +815,12 @@ void build_neighbours(fjsph_ctx* ctx, bool reorder)
         sync(ctx);
         if (ctx->sc_host->overflow) {
             /* a clustered region: shorter blocks have smaller unions */
-            if (ctx->tg.C > 1) {
-                set_tiles(std::max(1, ctx->tg.C / 2));
+            int k = 0;
+            for (int a = 1; a < D; ++a)
+                if (bc[a] >= bc[k]) k = a;
+            if (bc[k] > 1) {
+                bc[k] = bc[k] / 2;
+                set_tiles(bc);
                 continue;
             }
             throw std::string("neighbour candidate union of a one-cell tile block exceeds ") +
@@ -787,7 +832,7 @@ void build_neighbours(fjsph_ctx* ctx, bool reorder)
         if (mc <= ctx->nl.cap && ctx->nl.lu4) break;
         /* capacity in entries, a multiple of the 4-entry batch */
         const int32_t cap = ((mc + mc / 8 + 8) + 7) / 8 * 8;
-        dalloc(ctx->nl.lu4, size_t(cap / 4 + kRowSlack) * ctx->nl.npad + kTargetSlack);
+        dalloc(ctx->nl.lu4, size_t(cap / 4 + kRowSlack) * ctx->nl.npad);
         ctx->nl.cap = cap;
     }
     if (ctx->max_count > ctx->nl.cap) throw std::string("neighbour list capacity could not be established");

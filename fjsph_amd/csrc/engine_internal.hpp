@@ -67,22 +67,23 @@ constexpr int TILE = FJ_TILE;
 static_assert(TILE % 4 == 0, "tile slots come in groups of 4");
 constexpr uint32_t NO_ENTRY = 0xFFFF;
 /* Room past the list rows: the up to four waves that share a list load one
- * row each past its last one, and the lanes past a block's targets load the
- * positions after them (what they read is masked by the targets' row
- * counts). */
+ * row each past its last one (masked by the targets' row counts). */
 constexpr int kRowSlack = 4;
-constexpr int kTargetSlack = 256;
+/* Cell rows of a block's candidate union at most. */
+constexpr int kMaxRows = 25;
 /* Longest tile block in cells: every coordinate of a block's candidate
  * union then lies within 1000 H of its first target, the bound the FP32
  * prefilter of the list build relies on. */
 constexpr int32_t kMaxBlockCells = 256;
 
-/* Tile decomposition of the last neighbour build: block b covers cells
- * [q*C, q*C + C) of cell row b / nchunk, q = b % nchunk. */
+/* Tile decomposition of the last neighbour build: the blocks are boxes of
+ * bc cells along each axis (bc[k] = 1 along axes the dimension lacks),
+ * nb of them, x fastest. */
 struct TileGrid {
     int32_t dims[3];
-    int32_t C;
-    int32_t nchunk;
+    int32_t bc[3];
+    int32_t nb[3];
+    int32_t share;  /* waves of a short block share its lists (mixed precision) */
     int64_t nblocks;
     const int32_t* start; /* cell_start, ncell + 1 */
     const int32_t* order; /* slots in cell order (the candidate unions) */

@@ -1,11 +1,12 @@
 /*
  * Block-tiled pair passes of the WCSPH step.
  *
- * Work decomposition: a block is a chunk of C consecutive cells of one cell
- * row; its targets are the particles of those cells (positions [p0, p1) of
- * the cell-sorted order[] array, recorded as the target order vorder[]) and
- * its candidate union is the 3^(D-1) neighbour rows over cells
- * [cx0 - 1, cx1].  The union is staged in LDS in tiles of TILE records,
+ * Work decomposition: a block is a box of cells (TileGrid::bc along each
+ * axis); its targets are the particles of those cells (a run of positions
+ * of the cell-sorted order[] array per cell row, recorded as the target
+ * order vorder[]) and its candidate union is the box grown by one cell on
+ * every side, again one run of order[] per cell row.  The union is staged
+ * in LDS in tiles of TILE records,
  * dealt to the tiles round robin in groups of TGRP = 8 (tile_union_index); each
  * lane walks its own neighbour list tile by tile.  Pair terms never
  * scatter: every pass is owner-computes.
@@ -37,44 +38,93 @@
 
 namespace fj {
 
-constexpr int MAXSEG = 9;
+/* Threads of a block of the pair passes: four waves to a tile of 496
+ * records, five blocks a CU.  Eight waves to 992 records (two blocks a CU)
+ * have fuller rows and stage less per target, but wait longer at each tile's
+ * barriers: at 4M particles the step took 38.2 ms against 37.2, at 1M
+ * 14.5 against 14.3, at 200k in FP64 12.0 against 10.2. */
+constexpr int PTPB = 256;
+constexpr int PWAVE = PTPB / 64;
+static_assert(PWAVE == NWAVE, "block_reduce adds up NWAVE waves");
 
-/* Union of block b (see file header). seg_a[k] is the order[] start of
- * segment k, pre[k] its first union index; the target positions in order[]
- * are [p0, p1). */
+/* Cell rows of a block's candidate union at most (TileGrid::bc keeps to
+ * it), and the table's length: a power of two for the search. */
+constexpr int MAXSEG = kMaxRows;
+constexpr int SEGTAB = 32;
+static_assert(MAXSEG <= SEGTAB, "");
+
+/* Cells of block b along each axis: [c0, c1). */
 template <int D>
-__device__ void union_of_block(const TileGrid& tg, int64_t b, int32_t* seg_a, int32_t* pre, int& nseg, int& p0,
-                               int& p1)
+__device__ __forceinline__ void block_cells(const TileGrid& tg, int64_t b, int (&c0)[3], int (&c1)[3])
 {
-    const int64_t row = b / tg.nchunk;
-    const int q = (int)(b - row * tg.nchunk);
-    const int cx0 = q * tg.C;
-    const int cx1 = min(cx0 + tg.C, tg.dims[0]);
-    const int64_t rbase = row * tg.dims[0];
-    p0 = tg.start[rbase + cx0];
-    p1 = tg.start[rbase + cx1];
-    const int cy = (int)(row % tg.dims[1]);
-    const int cz = (D == 3) ? (int)(row / tg.dims[1]) : 0;
-    const int xa = max(cx0 - 1, 0), xb = min(cx1, tg.dims[0] - 1);
-    nseg = 0;
-    pre[0] = 0;
-    const int zlo = (D == 3) ? max(cz - 1, 0) : 0, zhi = (D == 3) ? min(cz + 1, tg.dims[2] - 1) : 0;
-    for (int z = zlo; z <= zhi; ++z)
-        for (int y = max(cy - 1, 0); y <= min(cy + 1, tg.dims[1] - 1); ++y) {
-            const int64_t r2 = ((int64_t)z * tg.dims[1] + y) * tg.dims[0];
-            const int32_t a = tg.start[r2 + xa], e = tg.start[r2 + xb + 1];
-            seg_a[nseg] = a;
-            pre[nseg + 1] = pre[nseg] + (e - a);
-            ++nseg;
-        }
+    const int64_t r = b / tg.nb[0];
+    const int q[3] = {int(b - r * tg.nb[0]), int(r % tg.nb[1]), int(r / tg.nb[1])};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        c0[k] = k < D ? q[k] * tg.bc[k] : 0;
+        c1[k] = k < D ? min(c0[k] + tg.bc[k], tg.dims[k]) : 1;
+    }
 }
 
-__device__ __forceinline__ int32_t union_slot(const TileGrid& tg, const int32_t* seg_a, const int32_t* pre, int nseg,
-                                              int u)
+/* The candidate union of a block: segment k holds order[] positions from
+ * seg_a[k] on and union indices [pre[k], pre[k + 1]); the table is filled
+ * up with empty segments. */
+struct UnionTab {
+    int32_t seg_a[SEGTAB];
+    int32_t pre[SEGTAB + 1];
+    int32_t nseg;
+};
+
+__device__ __forceinline__ int wave_incl_scan(int v, int lane)
+{
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(v, o, 64);
+        if (lane >= o) v += t;
+    }
+    return v;
+}
+
+/* Fills the union table of block b, one lane of the calling wave per row. */
+template <int D>
+__device__ __forceinline__ void union_of_block(const TileGrid& tg, int64_t b, UnionTab& ut)
+{
+    const int lane = threadIdx.x & 63;
+    int c0[3], c1[3];
+    block_cells<D>(tg, b, c0, c1);
+    const int ylo = max(c0[1] - 1, 0), ny = min(c1[1], tg.dims[1] - 1) - ylo + 1;
+    const int zlo = max(c0[2] - 1, 0), nz = min(c1[2], tg.dims[2] - 1) - zlo + 1;
+    const int xa = max(c0[0] - 1, 0), xe = min(c1[0], tg.dims[0] - 1) + 1;
+    int a = 0, len = 0;
+    if (lane < ny * nz) {
+        const int64_t r = (int64_t(zlo + lane / ny) * tg.dims[1] + (ylo + lane % ny)) * tg.dims[0];
+        a = tg.start[r + xa];
+        len = tg.start[r + xe] - a;
+    }
+    const int incl = wave_incl_scan(len, lane);
+    if (lane < SEGTAB) {
+        ut.seg_a[lane] = a;
+        ut.pre[lane + 1] = incl;
+    }
+    if (lane == 0) {
+        ut.pre[0] = 0;
+        ut.nseg = ny * nz;
+    }
+}
+
+/* order[] position of union index u (u below the union's size) */
+__device__ __forceinline__ int32_t union_pos(const UnionTab& ut, int u)
 {
     int k = 0;
-    while (k + 1 < nseg && u >= pre[k + 1]) ++k;
-    return tg.order[seg_a[k] + (u - pre[k])];
+#pragma unroll
+    for (int h = SEGTAB / 2; h > 0; h >>= 1)
+        if (ut.pre[k + h] <= u) k += h;
+    return ut.seg_a[k] + (u - ut.pre[k]);
+}
+
+__device__ __forceinline__ int32_t union_slot(const TileGrid& tg, const UnionTab& ut, int u)
+{
+    return tg.order[union_pos(ut, u)];
 }
 
 /* Union indices are dealt to the LDS tiles in groups of TGRP consecutive
@@ -115,44 +165,73 @@ __device__ __forceinline__ int entry_union_index(uint32_t e, int NT)
 __device__ __forceinline__ int64_t block_of_slot(const TileGrid& tg, int64_t i)
 {
     const int32_t lin = tg.cell[i];
-    const int64_t row = lin / tg.dims[0];
-    const int cx = lin - (int)(row * tg.dims[0]);
-    return row * tg.nchunk + cx / tg.C;
+    const int32_t row = lin / tg.dims[0];
+    const int cx = lin - row * tg.dims[0], cy = row % tg.dims[1], cz = row / tg.dims[1];
+    return (int64_t(cz / tg.bc[2]) * tg.nb[1] + cy / tg.bc[1]) * tg.nb[0] + cx / tg.bc[0];
 }
 
 /* Group of block b (independent simulations): the groups occupy disjoint
- * cell layers along the last axis, and a block lies in one cell row. */
+ * cell layers along the last axis, and a block then lies in one of them. */
 template <int D>
 __device__ __forceinline__ int32_t block_group(const TileGrid& tg, int64_t b)
 {
-    const int64_t row = b / tg.nchunk;
-    const int64_t layer = (D == 3) ? row / tg.dims[1] : row;
-    return tg.lgrp[layer];
+    const int64_t row = b / tg.nb[0];
+    return tg.lgrp[D == 3 ? row / tg.nb[1] : row];
 }
 
-/* Shared block prologue: union table in LDS, uniform p0/p1/U, and the
- * block b the workgroup runs. */
+/* Shared block prologue: union table and target runs in LDS, the numbers of
+ * targets T and of candidates U, a slot of the block (its first target: the
+ * reference point of relative coordinates), and the block b the workgroup
+ * runs. */
 struct BlockHead {
-    int32_t seg_a[MAXSEG];
-    int32_t pre[MAXSEG + 1];
-    int32_t nseg, p0, p1;
+    UnionTab ut;
+    int32_t tseg_a[MAXSEG];
+    int32_t tpre[MAXSEG + 1];
+    int32_t T, U, i0;
     int64_t b;
+    /* order[] position of target k of the block (k below T) */
+    __device__ __forceinline__ int target_pos(int k) const
+    {
+        int q = 0;
+        while (k >= tpre[q + 1]) ++q;
+        return tseg_a[q] + (k - tpre[q]);
+    }
 };
 
 template <int D>
 __device__ __forceinline__ void block_head(const TileGrid& tg, BlockHead& h)
 {
-    if (threadIdx.x == 0) {
-        int nseg, p0, p1;
+    if (threadIdx.x < 64) {
         /* workgroup w runs block w: dispatch order is cell order, so the
          * blocks in flight cover a band of neighbouring cell rows */
         const int64_t b = blockIdx.x;
-        h.b = b;
-        union_of_block<D>(tg, b, h.seg_a, h.pre, nseg, p0, p1);
-        h.nseg = nseg;
-        h.p0 = p0;
-        h.p1 = p1;
+        union_of_block<D>(tg, b, h.ut);
+        const int lane = threadIdx.x;
+        int c0[3], c1[3];
+        block_cells<D>(tg, b, c0, c1);
+        const int ny = c1[1] - c0[1], nz = c1[2] - c0[2];
+        int a = 0, len = 0;
+        if (lane < ny * nz) {
+            const int64_t r = (int64_t(c0[2] + lane / ny) * tg.dims[1] + (c0[1] + lane % ny)) * tg.dims[0];
+            a = tg.start[r + c0[0]];
+            len = tg.start[r + c1[0]] - a;
+        }
+        const int incl = wave_incl_scan(len, lane);
+        if (lane < MAXSEG) {
+            h.tseg_a[lane] = a;
+            h.tpre[lane + 1] = incl;
+        }
+        if (lane == 0) {
+            h.tpre[0] = 0;
+            h.b = b;
+        }
+        const uint64_t some = __ballot(len > 0);
+        const int first = some ? __ffsll((unsigned long long)some) - 1 : 0;
+        if (lane == first) h.i0 = len > 0 ? tg.order[a] : 0;
+        if (lane == 63) h.T = incl;
     }
+    __syncthreads();
+    if (threadIdx.x == 0) h.U = h.ut.pre[SEGTAB];
     __syncthreads();
 }
 
@@ -160,7 +239,7 @@ __device__ __forceinline__ void block_head(const TileGrid& tg, BlockHead& h)
  * threadIdx.x + TPB; -1 where there is none).  Loaded one tile ahead, so
  * the order[] lookup of the next tile is in flight while the current
  * tile's pairs run and staging after the barrier waits only for the data. */
-static_assert(TILE <= 2 * TPB, "a thread stages at most two slots per tile");
+static_assert(TILE <= 2 * PTPB, "a thread stages at most two slots per tile");
 struct TileSlots {
     int32_t sl[2];
     __device__ __forceinline__ void load(const TileGrid& tg, const BlockHead& h, int tk, int NT, int U)
@@ -168,15 +247,15 @@ struct TileSlots {
         const int nt = tk < NT ? tile_len(tk, U, NT) : 0;
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-            const int t = threadIdx.x + r * TPB;
+            const int t = threadIdx.x + r * PTPB;
             sl[r] = -1;
             if (t < nt) {
                 const int u = tile_union_index(tk, t, NT);
-                if (u < U) sl[r] = union_slot(tg, h.seg_a, h.pre, h.nseg, u);
+                if (u < U) sl[r] = union_slot(tg, h.ut, u);
             }
         }
     }
-    __device__ __forceinline__ int32_t at(int t) const { return t < TPB ? sl[0] : sl[1]; }
+    __device__ __forceinline__ int32_t at(int t) const { return t < PTPB ? sl[0] : sl[1]; }
 };
 
 /* x - ref as an FP32 value hi and its FP32 rounding residual lo (hi + lo
@@ -191,30 +270,34 @@ __device__ __forceinline__ void split_rel(double x, double ref, float& hi, float
     lo = float(d - double(hi));
 }
 
-/* How the waves of a block share its targets.  A block with more than two
- * waves' worth of targets gives each wave 64 of them; in a block with fewer
- * the waves left over take part in the same lists: `n` waves walk every
- * n-th row of the same 64 targets and their sums meet at the end
+/* How the waves of a block share its targets.  A block with more than half
+ * its waves' worth of targets gives each wave 64 of them; in a block with
+ * fewer the waves left over take part in the same lists: `n` waves walk
+ * every n-th row of the same 64 targets and their sums meet at the end
  * (split_fold).  A particle set that gives each CU less than a few blocks
- * runs on short blocks (build_neighbours) and so on four waves a list. */
+ * runs on short blocks (build_neighbours) and so on up to four waves a
+ * list.  Not in FP64 (TileGrid::share). */
 struct Split {
     int n, part, lane; /* waves to a list, this wave's place among them, the thread's target */
 };
 
-__device__ __forceinline__ Split split_of(const BlockHead& h)
+__device__ __forceinline__ Split split_of(const TileGrid& tg, const BlockHead& h)
 {
-    const int nw = __builtin_amdgcn_readfirstlane((h.p1 - h.p0 + 63) >> 6);
+    const int nw = __builtin_amdgcn_readfirstlane((h.T + 63) >> 6);
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     Split s;
-    s.n = nw <= 1 ? NWAVE : nw == 2 ? NWAVE / 2 : 1;
-    const int tw = NWAVE / s.n; /* waves with targets of their own */
+    s.n = 1;
+#pragma unroll
+    for (int k = PWAVE; k > 1; k >>= 1)
+        if (tg.share && s.n == 1 && nw * k <= PWAVE) s.n = k;
+    const int tw = PWAVE / s.n; /* waves with targets of their own */
     s.part = w / tw;
     s.lane = int(threadIdx.x) - s.part * tw * 64;
     return s;
 }
 
 /* Values of the waves of a list folded in wave order into the first one's;
- * `buf` is LDS of 3 TPB values that the block is done with. */
+ * `buf` is LDS of 3 PTPB values that the block is done with. */
 template <int N, typename Op>
 __device__ __forceinline__ void split_fold(const Split& sp, double (&v)[N], double* buf, Op op)
 {
@@ -223,17 +306,17 @@ __device__ __forceinline__ void split_fold(const Split& sp, double (&v)[N], doub
     for (int r = 0; r < N; r += 3) {
         __syncthreads();
 #pragma unroll
-        for (int k = r; k < (r + 3 < N ? r + 3 : N); ++k) buf[(k - r) * TPB + threadIdx.x] = v[k];
+        for (int k = r; k < (r + 3 < N ? r + 3 : N); ++k) buf[(k - r) * PTPB + threadIdx.x] = v[k];
         __syncthreads();
         if (sp.part == 0) {
-            const int step = TPB / sp.n;
+            const int step = PTPB / sp.n;
 #pragma unroll
             for (int k = r; k < (r + 3 < N ? r + 3 : N); ++k)
-                for (int q = 1; q < sp.n; ++q) v[k] = op(v[k], buf[(k - r) * TPB + threadIdx.x + q * step]);
+                for (int q = 1; q < sp.n; ++q) v[k] = op(v[k], buf[(k - r) * PTPB + threadIdx.x + q * step]);
         }
     }
 }
-static_assert(sizeof(float4) * TILE >= 3 * sizeof(double) * TPB, "a tile array serves as split_fold's buffer");
+static_assert(sizeof(double) * TILE * 2 >= 3 * sizeof(double) * PTPB, "a tile array of 16 B serves as split_fold's buffer");
 
 template <typename Op>
 __device__ __forceinline__ double split_fold1(const Split& sp, double v, double* buf, Op op)
@@ -251,7 +334,7 @@ __device__ __forceinline__ double split_fold1(const Split& sp, double v, double*
  * after them, at the end of the loop, was waited for at once: the loop
  * carries it in a register, and the copy into that register needs the
  * value).  The load has no branch: a lane reads on past its own nrows (the
- * array has kRowSlack rows and a block of targets to spare) and row_in()
+ * array has kRowSlack rows to spare) and row_in()
  * tells what counts.  Every lane with a list walks it, also a lane whose
  * target the pass does not compute (`on` false): the build pads each tile's
  * rows to the wave's largest count, and the wave leaves a tile only when no
@@ -388,24 +471,25 @@ __device__ __forceinline__ float wave_maxf(float v)
  * The test runs first in FP32 on coordinates relative to the block's first
  * target, each rounded once to FP32: with every coordinate within L of that
  * point, the FP32 squared distance near sr is off by at most about
- * 2^-23 (L / H) sr plus a few ulp, and L < (C + 2) cs sqrt(3) < 1000 H for
- * any tile grid (C <= 256 cells of size 2H), so below (1 - 1e-3) sr it is
+ * 2^-23 (L / H) sr plus a few ulp, and L < (bc + 2) cs sqrt(3) < 1000 H for
+ * any tile grid (at most 256 cells of size 2H along x, a few along the other
+ * axes), so below (1 - 1e-3) sr it is
  * surely in, above (1 + 1e-3) sr surely out, and only the thin shell
  * between is decided by the exact FP64 test.  The lists are those of the
  * FP64 test.  The candidate loop only marks what is not surely out; the
  * in/shell split and the FP64 test run on the marked ones (the ~240
  * neighbours of ~2000 candidates), in ascending order. */
 template <int D>
-__global__ __launch_bounds__(TPB) void k_build_t(const double* __restrict__ x, TileGrid tg, double sr, NbrList nl,
+__global__ __launch_bounds__(PTPB) void k_build_t(const double* __restrict__ x, TileGrid tg, double sr, NbrList nl,
                                                  DevScalars* sc)
 {
     __shared__ double tp[D][TILE];
     __shared__ float4 tf[(TILE + 31) / 32 * 32]; /* read in chunks of 32 */
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
-    if (h.p0 == h.p1) return;
+    if (h.T == 0) return;
     if (tg.gbuild) {
         /* a partial build (independent simulations): other groups keep
          * their lists */
@@ -418,15 +502,16 @@ __global__ __launch_bounds__(TPB) void k_build_t(const double* __restrict__ x, T
     }
     double xref[D];
     {
-        const int64_t i0 = tg.order[h.p0];
+        const int64_t i0 = h.i0;
 #pragma unroll
         for (int a = 0; a < D; ++a) xref[a] = x[i0 * D + a];
     }
     const float sr_lo = float(sr * (1.0 - 1e-3)), sr_hi = float(sr * (1.0 + 1e-3));
     const int rcap = nl.cap >> 2;
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + threadIdx.x;
-        const bool active = p < h.p1;
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const int k_t = kb + threadIdx.x;
+        const bool active = k_t < h.T;
+        const int p = h.target_pos(active ? k_t : 0);
         if (active) {
             const int32_t sl = tg.order[p];
             tg.vorder[p] = sl;
@@ -454,8 +539,10 @@ __global__ __launch_bounds__(TPB) void k_build_t(const double* __restrict__ x, T
         int k_self = -1, t_self = 0;
         if (active) {
             int sg = 0;
-            while (sg + 1 < h.nseg && !(p >= h.seg_a[sg] && p < h.seg_a[sg] + (h.pre[sg + 1] - h.pre[sg]))) ++sg;
-            const int u = h.pre[sg] + (p - h.seg_a[sg]);
+            while (sg + 1 < h.ut.nseg &&
+                   !(p >= h.ut.seg_a[sg] && p < h.ut.seg_a[sg] + (h.ut.pre[sg + 1] - h.ut.pre[sg])))
+                ++sg;
+            const int u = h.ut.pre[sg] + (p - h.ut.seg_a[sg]);
             const int g = u / TGRP;
             k_self = g % NT;
             t_self = (g / NT) * TGRP + u % TGRP;
@@ -465,14 +552,14 @@ __global__ __launch_bounds__(TPB) void k_build_t(const double* __restrict__ x, T
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int u = tile_union_index(tk, t, NT);
                 if (u >= U) {
                     /* padding: far away, never a neighbour */
                     tf[t] = make_float4(1e30f, 1e30f, 1e30f, -2.f);
                     continue;
                 }
-                const int32_t sl = union_slot(tg, h.seg_a, h.pre, h.nseg, u);
+                const int32_t sl = union_slot(tg, h.ut, u);
                 float pa[3] = {0.f, 0.f, 0.f};
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
@@ -485,10 +572,11 @@ __global__ __launch_bounds__(TPB) void k_build_t(const double* __restrict__ x, T
             /* groups of 4 slots with a candidate in reach of the wave's
              * box (squared distance to it at most sr_hi, which every
              * neighbour's FP32 squared distance to its target meets): one
-             * bit per group, wave-uniform (tiles hold at most 128 groups) */
-            uint64_t gmask[2];
+             * bit per group, wave-uniform */
+            constexpr int GW = (TILE / 4 + 63) / 64;
+            uint64_t gmask[GW];
 #pragma unroll
-            for (int hgrp = 0; hgrp < 2; ++hgrp) {
+            for (int hgrp = 0; hgrp < GW; ++hgrp) {
                 const int g = hgrp * 64 + (threadIdx.x & 63);
                 bool reach = false;
                 if (4 * g < nt) {
@@ -600,50 +688,69 @@ void launch_build_lists(int dim, const double* x, int64_t n, TileGrid tg, double
                         hipStream_t st)
 {
     (void)n;
-    const dim3 g((unsigned)tg.nblocks), b(TPB);
+    const dim3 g((unsigned)tg.nblocks), b(PTPB);
     if (dim == 2) hipLaunchKernelGGL(k_build_t<2>, g, b, 0, st, x, tg, sr, nl, sc);
     else hipLaunchKernelGGL(k_build_t<3>, g, b, 0, st, x, tg, sr, nl, sc);
 }
 
-/* f(j) for every neighbour slot j of slot i, one lane per slot (the passes
- * over the thin boundary layer and the host dump walk lists this way). */
+/* f(j) for every neighbour slot j of slot i, spread over the lanes of the
+ * wave (all lanes call it with the same i and the wave's own table). */
 template <int D, typename F>
-__device__ __forceinline__ void walk_lane(const TileGrid& tg, const NbrList& nl, int64_t i, F&& f)
+__device__ __forceinline__ void walk_wave(const TileGrid& tg, const NbrList& nl, UnionTab& ut, int64_t i, F&& f)
 {
-    int32_t seg_a[MAXSEG], pre[MAXSEG + 1];
-    int nseg, p0, p1;
-    union_of_block<D>(tg, block_of_slot(tg, i), seg_a, pre, nseg, p0, p1);
-    const int NT = n_tiles(pre[nseg]);
+    union_of_block<D>(tg, block_of_slot(tg, i), ut);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int NT = n_tiles(ut.pre[SEGTAB]);
     const int64_t p = tg.pos[i];
     const int nrows = min(nl.count[i], nl.cap >> 2);
-    for (int r = 0; r < nrows; ++r) {
+    for (int r = threadIdx.x & 63; r < nrows; r += 64) {
         const uint64_t u = nl.lu4[(int64_t)r * nl.npad + p];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const uint32_t uq = uint32_t(u >> (16 * q)) & 0xFFFFu;
-            if (uq != NO_ENTRY) f(union_slot(tg, seg_a, pre, nseg, entry_union_index(uq, NT)));
+            if (uq != NO_ENTRY) f(union_slot(tg, ut, entry_union_index(uq, NT)));
         }
     }
 }
 
 /* Global slots of every slot's neighbours, compacted: entry k of slot i at
- * out[k*npad + i] for k < nnb[i] (for the host dump of the lists). */
+ * out[k*npad + i] for k < nnb[i] (for the host dump of the lists), one wave
+ * per slot: a row's place is the number of entries of the rows before it. */
 template <int D>
 __global__ __launch_bounds__(TPB) void k_export(TileGrid tg, NbrList nl, int64_t n, int32_t* out)
 {
-    const int64_t i = blockIdx.x * (int64_t)TPB + threadIdx.x;
+    __shared__ UnionTab uts[NWAVE];
+    const int64_t i = (blockIdx.x * (int64_t)TPB + threadIdx.x) >> 6;
     if (i >= n) return;
-    int k = 0;
-    walk_lane<D>(tg, nl, i, [&](int32_t j) {
-        out[(int64_t)k * nl.npad + i] = j;
-        ++k;
-    });
+    UnionTab& ut = uts[threadIdx.x >> 6];
+    const int lane = threadIdx.x & 63;
+    union_of_block<D>(tg, block_of_slot(tg, i), ut);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int NT = n_tiles(ut.pre[SEGTAB]);
+    const int64_t p = tg.pos[i];
+    const int nrows = min(nl.count[i], nl.cap >> 2);
+    int base = 0;
+    for (int r0 = 0; r0 < nrows; r0 += 64) {
+        const uint64_t u = r0 + lane < nrows ? nl.lu4[(int64_t)(r0 + lane) * nl.npad + p] : ~0ull;
+        int cnt = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cnt += (uint32_t(u >> (16 * q)) & 0xFFFFu) != NO_ENTRY;
+        const int incl = wave_incl_scan(cnt, lane);
+        for (int q = 0; q < cnt; ++q) {
+            const uint32_t uq = uint32_t(u >> (16 * q)) & 0xFFFFu;
+            out[(int64_t)(base + incl - cnt + q) * nl.npad + i] = union_slot(tg, ut, entry_union_index(uq, NT));
+        }
+        base += __shfl(incl, 63, 64);
+    }
 }
 
 void launch_export_lists(int dim, TileGrid tg, NbrList nl, int64_t n, int32_t* out, hipStream_t st)
 {
-    if (dim == 2) hipLaunchKernelGGL(k_export<2>, dim3(grid_of(n)), dim3(TPB), 0, st, tg, nl, n, out);
-    else hipLaunchKernelGGL(k_export<3>, dim3(grid_of(n)), dim3(TPB), 0, st, tg, nl, n, out);
+    const dim3 g(grid_of(n * 64)), b(TPB);
+    if (dim == 2) hipLaunchKernelGGL(k_export<2>, g, b, 0, st, tg, nl, n, out);
+    else hipLaunchKernelGGL(k_export<3>, g, b, 0, st, tg, nl, n, out);
 }
 
 /* Distance of a pair as the reference uses it: sqrt of the d^2 of the last
@@ -763,23 +870,23 @@ __device__ __forceinline__ void dsph_out(DevState& s, Aux& ax, int64_t i, const 
  * colour function, and the per-block partial of npd.  k_dsph_fin turns
  * them into L^-1, the eigenvalues and the corrected gradients. */
 template <int D, bool FR>
-__global__ __launch_bounds__(TPB) void k_dsph_t(Consts c, DevState s, Aux ax, TileGrid tg, NbrList nl, double* partial)
+__global__ __launch_bounds__(PTPB) void k_dsph_t(Consts c, DevState s, Aux ax, TileGrid tg, NbrList nl, double* partial)
 {
     constexpr int NS = D * (D + 1) / 2;
     __shared__ double tp[D][TILE];
     __shared__ double tvol[TILE], trho[TILE];
     __shared__ int32_t tnb[TILE], tsl[FR ? TILE : 1];
     __shared__ BlockHead h;
-    __shared__ double lds[NWAVE];
+    __shared__ double lds[PWAVE];
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     double npd_acc = 0.0;
     const double inv_H = 1.0 / c.H;
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         double xi[D], xbi[D], Lm[NS], Lnb[NS], gR[D], nr[D];
 #pragma unroll
@@ -800,7 +907,7 @@ __global__ __launch_bounds__(TPB) void k_dsph_t(Consts c, DevState s, Aux ax, Ti
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
 #pragma unroll
@@ -839,20 +946,20 @@ __global__ __launch_bounds__(TPB) void k_dsph_t(Consts c, DevState s, Aux ax, Ti
 #define FJ_DSPH_OCC __attribute__((amdgpu_waves_per_eu(5, 8)))
 #endif
 template <int D, bool FR>
-__global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s, Aux ax, TileGrid tg, NbrList nl, double* partial)
+__global__ __launch_bounds__(PTPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s, Aux ax, TileGrid tg, NbrList nl, double* partial)
 {
     constexpr int NS = D * (D + 1) / 2;
     __shared__ float4 tA[TILE];            /* x_j - xref, +V_j (-V_j: j is PISTON or BOUND) */
     __shared__ float tR[TILE];             /* rho_j - rref */
     __shared__ float4 tX[FR ? TILE : 1];   /* xb_j - xbref */
     __shared__ BlockHead h;
-    __shared__ double lds[NWAVE];
+    __shared__ double lds[PWAVE];
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     double xref[D], xbref[D], rref;
     {
-        const int64_t i0 = tg.order[h.p0 < h.p1 ? h.p0 : 0];
+        const int64_t i0 = h.i0;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             xref[a] = s.x[i0 * D + a];
@@ -863,10 +970,10 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
     const float Ht = float(c.H), inv_Hf = float(1.0 / c.H), Wcf = float(c.Wc);
     const double inv_H = 1.0 / c.H;
     double npd_acc = 0.0;
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool slow = active && nl.nnb[i] < 2 * D;
         float xit[D], xlo[D], xbit[D], xblo[D];
@@ -891,7 +998,7 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
                 float pa[3] = {0.f, 0.f, 0.f}, xa[3] = {0.f, 0.f, 0.f};
@@ -999,7 +1106,7 @@ __global__ __launch_bounds__(TPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s
                 for (int q = 0; q < 4; ++q) {
                     const uint32_t e = uint32_t(e4 >> (16 * q)) & 0xFFFFu;
                     if (e == NO_ENTRY) continue;
-                    const int64_t j = union_slot(tg, h.seg_a, h.pre, h.nseg, entry_union_index(e, NT));
+                    const int64_t j = union_slot(tg, h.ut, entry_union_index(e, NT));
                     double xj[D], d2, rj;
 #pragma unroll
                     for (int a = 0; a < D; ++a) xj[a] = s.x[j * D + a];
@@ -1085,7 +1192,7 @@ __global__ __launch_bounds__(TPB) void k_dsph_fin(Consts c, DevState s, Aux ax, 
 void launch_dsph(int dim, const Consts& c, DevState s, Aux a, const int32_t* part_id, TileGrid tg, NbrList nl,
                  int64_t n, int r_from_x, int with_aero_vel, double* partial, DevScalars* sc, hipStream_t st)
 {
-    const dim3 g((unsigned)tg.nblocks), b(TPB);
+    const dim3 g((unsigned)tg.nblocks), b(PTPB);
     if (nl.f32) {
         if (dim == 2) {
             if (r_from_x) hipLaunchKernelGGL((k_dsph_m<2, false>), g, b, 0, st, c, s, a, tg, nl, partial);
@@ -1103,10 +1210,10 @@ void launch_dsph(int dim, const Consts& c, DevState s, Aux a, const int32_t* par
     }
     launch_sum_partials_scaled(partial, (int)tg.nblocks, 1, 1.0 / double(n), &sc->npd, st);
     if (dim == 2)
-        hipLaunchKernelGGL(k_dsph_fin<2>, dim3(grid_of(n)), b, 0, st, c, s, a, part_id, nl.nnb, n, with_aero_vel,
+        hipLaunchKernelGGL(k_dsph_fin<2>, dim3(grid_of(n)), dim3(TPB), 0, st, c, s, a, part_id, nl.nnb, n, with_aero_vel,
                            nl.f32);
     else
-        hipLaunchKernelGGL(k_dsph_fin<3>, dim3(grid_of(n)), b, 0, st, c, s, a, part_id, nl.nnb, n, with_aero_vel,
+        hipLaunchKernelGGL(k_dsph_fin<3>, dim3(grid_of(n)), dim3(TPB), 0, st, c, s, a, part_id, nl.nnb, n, with_aero_vel,
                            nl.f32);
 }
 
@@ -1254,7 +1361,7 @@ __device__ __forceinline__ void surface1_out(const Consts& c, DevState& s, int64
  * 2: dissipation_terms only.  T is the arithmetic of the dissipation terms
  * (FP32 on the mixed path). */
 template <int D, typename T, int MODE, bool FR>
-__global__ __launch_bounds__(TPB) void k_surface1_t(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
+__global__ __launch_bounds__(PTPB) void k_surface1_t(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
                                                     TileGrid tg, NbrList nl, double* norms_tmp)
 {
     constexpr bool with_surf = MODE != 2;
@@ -1265,15 +1372,15 @@ __global__ __launch_bounds__(TPB) void k_surface1_t(Consts c, DevState s, Aux ax
     __shared__ int32_t tnb[TD], tsl[FR ? TILE : 1];
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     const double inv_H = 1.0 / c.H;
     const double h133 = 1.33 * c.particle_step;
     const double r_lim = sqrt(2.0) * h133;
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
         double xi[D], xbi[D], ni[D], nhat[D], tau_hat[D], pT[D], vi[D], gri[D], nrm[D];
@@ -1315,7 +1422,7 @@ __global__ __launch_bounds__(TPB) void k_surface1_t(Consts c, DevState s, Aux ax
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
 #pragma unroll
@@ -1420,7 +1527,7 @@ __global__ __launch_bounds__(TPB) void k_surface1_t(Consts c, DevState s, Aux ax
 #define FJ_SURF1_OCC __attribute__((amdgpu_waves_per_eu(5, 8)))
 #endif
 template <int D, int MODE, bool FR>
-__global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
+__global__ __launch_bounds__(PTPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
                                                     TileGrid tg, NbrList nl, double* norms_tmp)
 {
     constexpr bool with_surf = MODE != 2;
@@ -1434,11 +1541,11 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
     __shared__ int32_t tsl[with_surf ? TILE : 1];
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     double xref[D], vref[D], xbref[D], rref;
     {
-        const int64_t i0 = tg.order[h.p0 < h.p1 ? h.p0 : 0];
+        const int64_t i0 = h.i0;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             xref[a] = s.x[i0 * D + a];
@@ -1455,10 +1562,10 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
     const float Ht = float(c.H), inv_H = float(1.0 / c.H), Wc = float(c.Wc);
     const float eps2 = float(0.0001 * c.H_sq), alpha = float(c.visc_alpha);
     const float rreff = float(rref);
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
         double nrm[D], av[D], rd = 0.0;
@@ -1518,7 +1625,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevSt
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
                 float pa[3] = {0.f, 0.f, 0.f}, va[3] = {0.f, 0.f, 0.f}, xa[3] = {0.f, 0.f, 0.f};
@@ -1712,6 +1819,7 @@ __global__ void k_clear_count(int32_t* count) { *count = 0; }
 template <int D, bool FR>
 __global__ __launch_bounds__(TPB) void k_surface1_resolve(Consts c, DevState s, Aux ax, TileGrid tg, NbrList nl)
 {
+    __shared__ UnionTab uts[NWAVE];
     const int32_t cnt = ax.sund[0];
     const int lane = threadIdx.x & 63;
     const int64_t nwave = int64_t(gridDim.x) * (TPB / 64);
@@ -1726,20 +1834,9 @@ __global__ __launch_bounds__(TPB) void k_surface1_resolve(Consts c, DevState s, 
                 found = marrone_exact<D, FR>(c, s, ax, i, sl);
             }
         } else {
-            int32_t seg_a[MAXSEG], pre[MAXSEG + 1];
-            int nseg, p0, p1;
-            union_of_block<D>(tg, block_of_slot(tg, i), seg_a, pre, nseg, p0, p1);
-            const int NT = n_tiles(pre[nseg]);
-            const int64_t p = tg.pos[i];
-            const int nrows = min(nl.count[i], nl.cap >> 2);
-            for (int r = lane; r < nrows && !found; r += 64) {
-                const uint64_t u = nl.lu4[(int64_t)r * nl.npad + p];
-                for (int q = 0; q < 4 && !found; ++q) {
-                    const uint32_t uq = uint32_t(u >> (16 * q)) & 0xFFFFu;
-                    if (uq != NO_ENTRY)
-                        found = marrone_exact<D, FR>(c, s, ax, i, union_slot(tg, seg_a, pre, nseg, entry_union_index(uq, NT)));
-                }
-            }
+            walk_wave<D>(tg, nl, uts[threadIdx.x >> 6], i, [&](int32_t j) {
+                if (!found) found = marrone_exact<D, FR>(c, s, ax, i, j);
+            });
         }
         found = __any(found);
         if (lane == 0) s.surf[i] = found ? 0 : 1;
@@ -1750,7 +1847,7 @@ template <int D, typename T, int MODE>
 static void launch_surface1_m(const Consts& c, DevState s, Aux a, const int32_t* part_id, TileGrid tg, NbrList nl,
                               int64_t n, int r_from_x, double* norms_tmp, hipStream_t st)
 {
-    const dim3 g((unsigned)tg.nblocks), b(TPB);
+    const dim3 g((unsigned)tg.nblocks), b(PTPB);
     if constexpr (sizeof(T) == 4) {
         if constexpr (MODE != 2) hipLaunchKernelGGL(k_clear_count, dim3(1), dim3(1), 0, st, a.sund);
         if (r_from_x)
@@ -1794,7 +1891,7 @@ void launch_surface1(int dim, int prec, const Consts& c, DevState s, Aux a, cons
 
 /* Curvature, Gissler occlusion and surfzone (src/Geometry.cpp:145-277). */
 template <int D, bool FR>
-__global__ __launch_bounds__(TPB) void k_surface2_t(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
+__global__ __launch_bounds__(PTPB) void k_surface2_t(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
                                                     TileGrid tg, NbrList nl, const double* __restrict__ norms_tmp)
 {
     __shared__ double tp[D][TILE], tn[D][TILE];
@@ -1802,13 +1899,13 @@ __global__ __launch_bounds__(TPB) void k_surface2_t(Consts c, DevState s, Aux ax
     __shared__ int32_t tsurf[TILE], tsl[FR ? TILE : 1];
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     const double inv_H = 1.0 / c.H;
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
         double xi[D], xbi[D], ni[D], Vd[D], Li[D][D];
@@ -1839,7 +1936,7 @@ __global__ __launch_bounds__(TPB) void k_surface2_t(Consts c, DevState s, Aux ax
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
 #pragma unroll
@@ -1911,7 +2008,7 @@ __global__ __launch_bounds__(TPB) void k_surface2_t(Consts c, DevState s, Aux ax
 #define FJ_SURF2_OCC __attribute__((amdgpu_waves_per_eu(5, 8)))
 #endif
 template <int D, bool FR>
-__global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
+__global__ __launch_bounds__(PTPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
                                                     TileGrid tg, NbrList nl, const double* __restrict__ norms_tmp)
 {
     __shared__ float4 tA[TILE];            /* x_j - xref, V_j */
@@ -1919,11 +2016,11 @@ __global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevSt
     __shared__ float4 tX[FR ? TILE : 1];   /* xb_j - xbref */
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     double xref[D], xbref[D];
     {
-        const int64_t i0 = tg.order[h.p0 < h.p1 ? h.p0 : 0];
+        const int64_t i0 = h.i0;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             xref[a] = s.x[i0 * D + a];
@@ -1931,10 +2028,10 @@ __global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevSt
         }
     }
     const float Ht = float(c.H), inv_Hf = float(1.0 / c.H), Wcf = float(c.Wc);
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
         float xit[D], xlo[D], xbit[D], xblo[D], ni[D], Vd[D], Li[D][D];
@@ -1972,7 +2069,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevSt
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
                 float pa[3] = {0.f, 0.f, 0.f}, na[3] = {0.f, 0.f, 0.f}, xa[3] = {0.f, 0.f, 0.f};
@@ -2076,7 +2173,7 @@ void launch_surface2(int dim, const Consts& c, DevState s, Aux a, const int32_t*
                      int64_t n, int r_from_x, const double* norms_tmp, hipStream_t st)
 {
     (void)n;
-    const dim3 g((unsigned)tg.nblocks), b(TPB);
+    const dim3 g((unsigned)tg.nblocks), b(PTPB);
     if (nl.f32) {
         if (dim == 2) {
             if (r_from_x) hipLaunchKernelGGL((k_surface2_m<2, false>), g, b, 0, st, c, s, a, part_id, tg, nl, norms_tmp);
@@ -2145,7 +2242,7 @@ __device__ __forceinline__ void shift_out(const Consts& c, DevState& s, int64_t 
  * win the reference's max and acos is decreasing, so the result is the same.
  * max_j |v_j - v_i| is taken on squared norms. */
 template <int D, bool FR>
-__global__ __launch_bounds__(TPB) void k_shift_t(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
+__global__ __launch_bounds__(PTPB) void k_shift_t(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
                                                  TileGrid tg, NbrList nl)
 {
     __shared__ double tp[D][TILE], tv[D][TILE], tn[D][TILE];
@@ -2153,14 +2250,14 @@ __global__ __launch_bounds__(TPB) void k_shift_t(Consts c, DevState s, Aux ax, c
     __shared__ int32_t tnb[TILE], tsl[FR ? TILE : 1];
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     const double inv_H = 1.0 / c.H;
     const double inv_Wdx = 1.0 / c.W_dx;
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
         const double lam_nb = fluid ? s.lam_nb[i] : 0.0;
@@ -2182,7 +2279,7 @@ __global__ __launch_bounds__(TPB) void k_shift_t(Consts c, DevState s, Aux ax, c
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
 #pragma unroll
@@ -2239,7 +2336,7 @@ __global__ __launch_bounds__(TPB) void k_shift_t(Consts c, DevState s, Aux ax, c
 #define FJ_SHIFT_OCC __attribute__((amdgpu_waves_per_eu(5, 8)))
 #endif
 template <int D, bool FR>
-__global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
+__global__ __launch_bounds__(PTPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
                                                  TileGrid tg, NbrList nl)
 {
     __shared__ float4 tA[TILE];            /* x_j - xref, +V_j (-V_j: j is PISTON or BOUND) */
@@ -2248,11 +2345,11 @@ __global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState
     __shared__ float4 tX[FR ? TILE : 1];   /* xb_j - xbref */
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     double xref[D], vref[D], xbref[D];
     {
-        const int64_t i0 = tg.order[h.p0 < h.p1 ? h.p0 : 0];
+        const int64_t i0 = h.i0;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             xref[a] = s.x[i0 * D + a];
@@ -2261,10 +2358,10 @@ __global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState
         }
     }
     const float Ht = float(c.H), inv_Hf = float(1.0 / c.H), Wcf = float(c.Wc), inv_Wdx = float(1.0 / c.W_dx);
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
         const double lam_nb = fluid ? s.lam_nb[i] : 0.0;
@@ -2289,7 +2386,7 @@ __global__ __launch_bounds__(TPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
                 float pa[3] = {0.f, 0.f, 0.f}, va[3] = {0.f, 0.f, 0.f}, xa[3] = {0.f, 0.f, 0.f};
@@ -2380,7 +2477,7 @@ void launch_shift(int dim, const Consts& c, DevState s, Aux a, const int32_t* pa
                   int64_t n, int r_from_x, hipStream_t st)
 {
     (void)n;
-    const dim3 g((unsigned)tg.nblocks), b(TPB);
+    const dim3 g((unsigned)tg.nblocks), b(PTPB);
     if (nl.f32) {
         if (dim == 2) {
             if (r_from_x) hipLaunchKernelGGL((k_shift_m<2, false>), g, b, 0, st, c, s, a, part_id, tg, nl);
@@ -2416,7 +2513,7 @@ void launch_shift(int dim, const Consts& c, DevState s, Aux a, const int32_t* pa
 #define FJ_SURF2SHIFT_OCC __attribute__((amdgpu_waves_per_eu(4, 8)))
 #endif
 template <int D, bool FR>
-__global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts c, DevState s, Aux ax,
+__global__ __launch_bounds__(PTPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts c, DevState s, Aux ax,
                                                                    const int32_t* __restrict__ part_id, TileGrid tg,
                                                                    NbrList nl, const double* __restrict__ norms_tmp)
 {
@@ -2427,11 +2524,11 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
     __shared__ float4 tX[FR ? TILE : 1];   /* xb_j - xbref */
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     double xref[D], vref[D], xbref[D];
     {
-        const int64_t i0 = tg.order[h.p0 < h.p1 ? h.p0 : 0];
+        const int64_t i0 = h.i0;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             xref[a] = s.x[i0 * D + a];
@@ -2447,10 +2544,10 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
      * is 1e-5 */
     const double cos15 = cos(kPi / 12.0);
     const float ang_yes_lo = float(-1.0 + 1e-5), ang_yes_hi = float(cos15 - 1e-5), ang_no = float(cos15 + 1e-5);
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
         const double lam_nb = fluid ? s.lam_nb[i] : 0.0;
@@ -2496,7 +2593,7 @@ __global__ __launch_bounds__(TPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts 
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
                 float pa[3] = {0.f, 0.f, 0.f}, va[3] = {0.f, 0.f, 0.f}, na[3] = {0.f, 0.f, 0.f},
@@ -2655,7 +2752,7 @@ void launch_surface2_shift(int dim, const Consts& c, DevState s, Aux a, const in
                            NbrList nl, int64_t n, int r_from_x, const double* norms_tmp, hipStream_t st)
 {
     (void)n;
-    const dim3 g((unsigned)tg.nblocks), b(TPB);
+    const dim3 g((unsigned)tg.nblocks), b(PTPB);
     if (dim == 2) {
         if (r_from_x) hipLaunchKernelGGL((k_surf2_shift_m<2, false>), g, b, 0, st, c, s, a, part_id, tg, nl, norms_tmp);
         else hipLaunchKernelGGL((k_surf2_shift_m<2, true>), g, b, 0, st, c, s, a, part_id, tg, nl, norms_tmp);
@@ -2680,34 +2777,18 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-/* f(j, r) for every neighbour j of slot i, spread over the lanes of the
- * wave (all lanes call it with the same i); r is the distance of the last
- * build. */
+/* walk_wave with the distance r of the last build. */
 template <int D, typename F>
 __device__ __forceinline__ void walk_wave_r(const TileGrid& tg, const NbrList& nl, const double* __restrict__ xb,
-                                            int64_t i, F&& f)
+                                            UnionTab& ut, int64_t i, F&& f)
 {
-    const int lane = threadIdx.x & 63;
-    int32_t seg_a[MAXSEG], pre[MAXSEG + 1];
-    int nseg, p0, p1;
-    union_of_block<D>(tg, block_of_slot(tg, i), seg_a, pre, nseg, p0, p1);
-    const int NT = n_tiles(pre[nseg]);
-    const int64_t p = tg.pos[i];
-    const int nrows = min(nl.count[i], nl.cap >> 2);
     double xbi[D];
     load_vec<D>(xb, i, xbi);
-    for (int r = lane; r < nrows; r += 64) {
-        const uint64_t u = nl.lu4[(int64_t)r * nl.npad + p];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t uq = uint32_t(u >> (16 * q)) & 0xFFFFu;
-            if (uq == NO_ENTRY) continue;
-            const int32_t j = union_slot(tg, seg_a, pre, nseg, entry_union_index(uq, NT));
-            double xbj[D];
-            load_vec<D>(xb, j, xbj);
-            f(j, sqrt(exact_dist2<D>(xbi, xbj)));
-        }
-    }
+    walk_wave<D>(tg, nl, ut, i, [&](int32_t j) {
+        double xbj[D];
+        load_vec<D>(xb, j, xbj);
+        f(j, sqrt(exact_dist2<D>(xbi, xbj)));
+    });
 }
 
 /* The slots of boundary block `block`, appended (count at out[0]). */
@@ -2730,6 +2811,7 @@ template <int D>
 __global__ __launch_bounds__(TPB) void k_bnd_vel(Consts c, DevState s, Aux ax, DevBlocks bl, int32_t block,
                                                  TileGrid tg, NbrList nl, const int32_t* __restrict__ slots)
 {
+    __shared__ UnionTab uts[NWAVE];
     const int64_t i = wave_slot(slots);
     if (i < 0) return;
     double v[D];
@@ -2741,7 +2823,7 @@ __global__ __launch_bounds__(TPB) void k_bnd_vel(Consts c, DevState s, Aux ax, D
 #pragma unroll
         for (int a = 0; a < D; ++a) vs[a] = 0.0;
         double ks = 0.0;
-        walk_wave_r<D>(tg, nl, ax.xb, i, [&](int32_t j, double r) {
+        walk_wave_r<D>(tg, nl, ax.xb, uts[threadIdx.x >> 6], i, [&](int32_t j, double r) {
             if (s.b[j] <= FJSPH_PISTON) return;
             double W, fg;
             wendland<double>(r, c.H, inv_H, c.Wc, W, fg);
@@ -2770,6 +2852,7 @@ __global__ __launch_bounds__(TPB) void k_bnd_solve(Consts c, DevState s, Aux ax,
                                                    TileGrid tg, NbrList nl, const int32_t* __restrict__ slots,
                                                    int32_t* near_inlet)
 {
+    __shared__ UnionTab uts[NWAVE];
     const int64_t i = wave_slot(slots);
     if (i < 0) return;
     const bool lead = (threadIdx.x & 63) == 0;
@@ -2787,7 +2870,7 @@ __global__ __launch_bounds__(TPB) void k_bnd_solve(Consts c, DevState s, Aux ax,
         double ks = 0.0, pk = 0.0, ak[D];
 #pragma unroll
         for (int a = 0; a < D; ++a) ak[a] = 0.0;
-        walk_wave_r<D>(tg, nl, ax.xb, i, [&](int32_t j, double r) {
+        walk_wave_r<D>(tg, nl, ax.xb, uts[threadIdx.x >> 6], i, [&](int32_t j, double r) {
             if (s.b[j] <= FJSPH_PISTON) return;
             double W, fg;
             wendland<double>(r, c.H, inv_H, c.Wc, W, fg);
@@ -2820,7 +2903,7 @@ __global__ __launch_bounds__(TPB) void k_bnd_solve(Consts c, DevState s, Aux ax,
         int ni = 1;
         double rr = 0.0, vi[D];
         load_vec<D>(s.v, i, vi);
-        walk_wave_r<D>(tg, nl, ax.xb, i, [&](int32_t j, double r) {
+        walk_wave_r<D>(tg, nl, ax.xb, uts[threadIdx.x >> 6], i, [&](int32_t j, double r) {
             const int32_t bj = s.b[j];
             if (bj == FJSPH_PIPE || bj == FJSPH_FREE) ni = 0;
             double W, fg;
@@ -3012,10 +3095,12 @@ __device__ void skin_friction(const Consts& c, const double* Vd, const double* n
 }
 
 
-/* Occupancy request for the force passes: 5 waves per SIMD (at most 102
- * VGPRs) measured faster than the compiler's 4 at 97 VGPRs. */
+/* Occupancy request for the force passes: four waves per SIMD.  With two
+ * records in flight the pass is bound by vector issue (0.94 instructions per
+ * CU-cycle at 4M particles), and a fifth wave only spills: 2.57 ms a launch
+ * against 2.74. */
 #ifndef FJ_FORCE_OCC
-#define FJ_FORCE_OCC __attribute__((amdgpu_waves_per_eu(5, 8)))
+#define FJ_FORCE_OCC __attribute__((amdgpu_waves_per_eu(4, 8)))
 #endif
 
 /* LDS tile of the FP64 force pass (parity path), one array per value: x, m,
@@ -3037,14 +3122,14 @@ struct ForceTile {
  * acc_i = sum_j (visc + ST / m_i - m_j (P_i + P_j) g).
  * FR: the positions have moved since the build, r comes from Aux::xb. */
 template <int D, bool FR>
-__global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_t(Consts c, DevState s, Aux ax,
+__global__ __launch_bounds__(PTPB) FJ_FORCE_OCC void k_force_t(Consts c, DevState s, Aux ax,
                                                               const int32_t* __restrict__ part_id, TileGrid tg,
                                                               NbrList nl, const DevScalars* sc)
 {
     __shared__ ForceTile<FR> ft;
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     double npd = sc->npd;
     if (tg.lgrp) {
@@ -3060,10 +3145,10 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_t(Consts c, DevState
     const double eps2 = 0.001 * c.H_sq;
     const double nu = c.nu;
     const double contang_fac = 1.0 + 0.5 * cos(0.5 * kPi * 7.0 / 9.0);
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
         double xi[D], vi[D], xbi[D], vpi[D];
@@ -3092,7 +3177,7 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_t(Consts c, DevState
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
 #pragma unroll
@@ -3209,7 +3294,7 @@ struct ForceTileM {
  * a_j and S = sum_j V_j g, and vPert_i . S enters the three sums once per
  * target. */
 template <int D, bool FR, bool ALE>
-__global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState s, Aux ax,
+__global__ __launch_bounds__(PTPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState s, Aux ax,
                                                               const int32_t* __restrict__ part_id, TileGrid tg,
                                                               NbrList nl, const DevScalars* sc)
 {
@@ -3217,13 +3302,13 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
     __shared__ ForceTileM<ALE> ft;
     __shared__ BlockHead h;
     block_head<D>(tg, h);
-    const int U = h.pre[h.nseg];
+    const int U = h.U;
     const int NT = n_tiles(U);
     /* reference point of the block (its first target) for the FP32
      * relative coordinates */
     double xref[D], vref[D], xbref[D];
     {
-        const int64_t i0 = tg.order[h.p0 < h.p1 ? h.p0 : 0];
+        const int64_t i0 = h.i0;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             xref[a] = s.x[i0 * D + a];
@@ -3248,10 +3333,10 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
     const float eps2 = float(0.001 * c.H_sq);
     const float nu = float(c.nu);
     const float contang_fac = float(1.0 + 0.5 * cos(0.5 * kPi * 7.0 / 9.0));
-    const Split sp = split_of(h);
-    for (int pb = h.p0; pb < h.p1; pb += TPB) {
-        const int p = pb + sp.lane;
-        const bool active = p < h.p1;
+    const Split sp = split_of(tg, h);
+    for (int kb = 0; kb < h.T; kb += PTPB) {
+        const bool active = kb + sp.lane < h.T;
+        const int p = h.target_pos(active ? kb + sp.lane : 0);
         const int64_t i = active ? tg.vorder[p] : 0;
         const bool fluid = active && part_id[i] >= c.n_bound;
         float xit[D], xlo[D], vit[D], vlo[D], xbit[D], xblo[D], vpi[D];
@@ -3283,7 +3368,7 @@ __global__ __launch_bounds__(TPB) FJ_FORCE_OCC void k_force_m(Consts c, DevState
         for (int tk = 0, base = 0; tk < NT; ++tk, base += TILE) {
             const int nt = tile_len(tk, U, NT);
             __syncthreads();
-            for (int t = threadIdx.x; t < nt; t += TPB) {
+            for (int t = threadIdx.x; t < nt; t += PTPB) {
                 const int32_t sl = ts.at(t);
                 if (sl < 0) continue;
                 float pa[3] = {0.f, 0.f, 0.f}, va[3] = {0.f, 0.f, 0.f}, xa[3] = {0.f, 0.f, 0.f};
@@ -3696,7 +3781,7 @@ void launch_sqdiff(int dim, const double* xa, const double* xb, const int32_t* p
 void launch_force(int dim, const Consts& c, DevState s, Aux a, const int32_t* part_id, TileGrid tg, NbrList nl,
                   int r_from_x, const DevScalars* sc, hipStream_t st)
 {
-    const dim3 g((unsigned)tg.nblocks), b(TPB);
+    const dim3 g((unsigned)tg.nblocks), b(PTPB);
 #define FJ_FORCE_T(DD, FF) hipLaunchKernelGGL((k_force_t<DD, FF>), g, b, 0, st, c, s, a, part_id, tg, nl, sc)
 #define FJ_FORCE_M(DD, FF, AA) hipLaunchKernelGGL((k_force_m<DD, FF, AA>), g, b, 0, st, c, s, a, part_id, tg, nl, sc)
 #define FJ_FORCE_MA(DD, FF) \

@@ -369,9 +369,10 @@ fjsph_status fjsph_get_group_info(fjsph_ctx* ctx, int32_t first, int32_t count, 
 
 /* Targets per tile block of the pair passes (the cells of one block row
  * whose particles share one candidate union in LDS); 0 restores the
- * default, 256, or 128 or 64 while the particle set is too small to fill
- * the device with blocks of 256 (reported as 256).  No counterpart in the reference.  Results change only in
- * the order of summation.  A block spans at most 256 cells whatever the
+ * default: 256, or in mixed precision 128 or 64 while the particle set is
+ * too small to fill the device with blocks of 256 (reported as 256).  No
+ * counterpart in the reference.  Results change only in the order of
+ * summation.  A block spans at most 256 cells whatever the
  * setting, and a block whose candidate union overflows the 16-bit list
  * entries (a clustered region) makes the build halve the block length
  * and try again, down to one cell. */

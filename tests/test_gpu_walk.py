@@ -83,8 +83,9 @@ def test_row_remainders(dim, ale, sizes, precision):
 @pytest.mark.parametrize("targets", [16, 64, 128, 192])
 @pytest.mark.parametrize("name", ["dam2d", "jet3d_ale", "drop3d"])
 def test_shared_lists(name, targets, precision):
-    """Start-up pass and two steps with blocks of few targets: four waves to
-    a list (16, 64), two (128), one (192), and a run's mixture of them."""
+    """Start-up pass and two steps with blocks of few targets: in mixed
+    precision four waves to a list (16, 64), two (128), one (192), and a run's
+    mixture of them."""
     case = dict(_small_cases())[name]
     case.settings.precision = precision
     print(f"[walk] {name}: n={case.n} {targets} targets a block, precision={precision}", flush=True)
@@ -100,4 +101,38 @@ def test_shared_lists(name, targets, precision):
     assert np.array_equal(eng.field("SURF"), orc.field("SURF"))
     for f in ("X", "V", "RHO", "ACC", "RRHO", "LAM", "AVISC"):
         assert_close(f, eng.field(f), orc.field(f), tol)
+    eng.close()
+
+
+@pytest.mark.parametrize("precision", [abi.PREC_FP64, abi.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("targets", [0, 8, 70, 512])
+@pytest.mark.parametrize("cells", [(9, 1), (1, 9), (12, 9), (300, 2), (7, 1, 1), (1, 1, 7), (2, 9, 1), (5, 4, 6)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_block_shapes(cells, targets, precision):
+    """Neighbour sets for clouds of every aspect (cut-off cells along the
+    axes), blocks of one cell to the whole cloud.  Half the particles lie on
+    a lattice whose step divides the cut-off, so that some pairs are a
+    rounding from it on either side."""
+    dim, dx = len(cells), 1e-3
+    c = cases.fluid_block(dim, 2, dx=dx, precision=precision, H_fac=2.0, sig=0.07)
+    rng = np.random.default_rng(5)
+    step = dx * (dim - 1)
+    g = np.stack(np.meshgrid(*[np.arange(max(1, round((4 * k - 1) * dx / step))) for k in cells], indexing="ij"), -1)
+    g = g.reshape(-1, dim) * step
+    loose = rng.random(len(g)) < 0.5
+    g[loose] += rng.uniform(-0.4, 0.4, (loose.sum(), dim)) * step
+    c.x = np.ascontiguousarray(g[rng.permutation(len(g))])
+    n = len(c.x)
+    c.v, c.rho, c.p = np.zeros((n, dim)), np.full(n, c.settings.rho_rest), np.zeros(n)
+    c.m, c.b = np.full(n, c.settings.rho_rest * dx ** dim), np.full(n, abi.FREE, dtype=np.int32)
+    c.n_bound, c.blocks = 0, [dict(first=0, last=n, is_fluid=1)]
+    print(f"[walk] cells {cells} n={n} {targets} targets a block, precision={precision}", flush=True)
+    eng, orc = _engine(c), _oracle(c)
+    eng.set_block_targets(targets)
+    eng.build_neighbours()
+    orc.build_neighbours()
+    off_e, idx_e = eng.neighbours()
+    off_o, idx_o, _ = orc.neighbours()
+    assert same_neighbour_sets(off_e, idx_e, off_o, idx_o)
+    assert np.array_equal(eng.neighbour_counts(), np.diff(off_e))
     eng.close()
