@@ -3216,22 +3216,13 @@ struct TrainBufs {
 int64_t mlp_nw(int D, int L) { return int64_t(64) * D + int64_t(L - 1) * 64 * 64 + int64_t(D + 2) * 64; }
 int64_t mlp_nb(int D, int L) { return int64_t(L) * 64 + D + 2; }
 
-/* One forward/backward pass over the batch idx (on the device) with the
- * parameters p (weights then biases): gradients into g, the batch's sum of
- * squared errors into *sse (device). */
-void mlp_pass(fjsph_ctx* ctx, MlpTrain& m, float* p, float* g, float* sse, void* wf, void* wt)
+/* The parameters p (weights then biases) and their tiles in a pass. */
+void mlp_params(MlpTrain& m, float* p, void* wf, void* wt)
 {
-    const int D = ctx->s.dim, L = m.n_hidden;
-    const int64_t nwaves = m.batch / 64;
-    launch_mlp_pack(D, p, L, wf, wt, ctx->st);
     m.wf = wf;
     m.wt = wt;
     m.b = p + m.nw;
-    m.bo = p + m.nw + int64_t(L) * 64;
-    launch_mlp_train(D, m, ctx->st);
-    launch_mlp_reduce(m.dWp, nwaves, m.nw, m.nw, g, ctx->st);
-    launch_mlp_reduce(m.dbp, nwaves, m.nb, m.nb, g + m.nw, ctx->st);
-    launch_mlp_reduce(m.lossp, nwaves, 1, 1, sse, ctx->st);
+    m.bo = p + m.nw + int64_t(m.n_hidden) * 64;
 }
 
 /* Scratch of a pass over a batch of B samples. */
@@ -3243,7 +3234,6 @@ void mlp_scratch(TrainBufs& tb, MlpTrain& m, int D, int L, int32_t B)
     m.nb = mlp_nb(D, L);
     const int64_t nwaves = B / 64;
     m.Z = tb.alloc<float>(size_t(L) * B * 64);
-    m.H = tb.alloc<__bf16>(size_t(L + 1) * B * 64);
     m.dWp = tb.alloc<float>(size_t(nwaves) * m.nw);
     m.dbp = tb.alloc<float>(size_t(nwaves) * m.nb);
     m.lossp = tb.alloc<float>(size_t(nwaves));
@@ -3288,7 +3278,10 @@ fjsph_status fjsph_surrogate_grad(fjsph_ctx* ctx, int32_t n_hidden, int32_t batc
         m.X = dX;
         m.T = dT;
         m.idx = didx;
-        mlp_pass(ctx, m, p, g, sse, wf, wt);
+        mlp_params(m, p, wf, wt);
+        launch_mlp_pack(D, p, L, wf, wt, ctx->st);
+        launch_mlp_train(D, m, ctx->st);
+        launch_mlp_reduce(m, g, g + m.nw, sse, ctx->st);
         sync(ctx);
         HIPCHK(hipMemcpy(dweights, g, size_t(m.nw) * 4, hipMemcpyDeviceToHost));
         HIPCHK(hipMemcpy(dbiases, g + m.nw, size_t(m.nb) * 4, hipMemcpyDeviceToHost));
@@ -3331,7 +3324,6 @@ fjsph_status fjsph_surrogate_grad_noalloc(fjsph_ctx* ctx, int32_t n_hidden, int3
         float* T = (float*)carve(size_t(batch) * 8 * sizeof(float));
         int32_t* idx = (int32_t*)carve(size_t(batch) * sizeof(int32_t));
         m.Z = (float*)carve(size_t(L) * batch * 64 * sizeof(float));
-        m.H = (__bf16*)carve(size_t(L + 1) * batch * 64 * sizeof(__bf16));
         m.dWp = (float*)carve(size_t(nwaves) * m.nw * sizeof(float));
         m.dbp = (float*)carve(size_t(nwaves) * m.nb * sizeof(float));
         m.lossp = (float*)carve(size_t(nwaves) * sizeof(float));
@@ -3350,12 +3342,8 @@ fjsph_status fjsph_surrogate_grad_noalloc(fjsph_ctx* ctx, int32_t n_hidden, int3
         m.b = biases;
         m.bo = biases + int64_t(L) * 64;
         launch_mlp_train(D, m, ctx->st);
-        launch_mlp_reduce(m.dWp, nwaves, m.nw, m.nw, dweights, ctx->st);
-        launch_mlp_reduce(m.dbp, nwaves, m.nb, m.nb, dbiases, ctx->st);
-        if (loss) {
-            launch_mlp_reduce(m.lossp, nwaves, 1, 1, sse, ctx->st);
-            launch_mlp_loss(sse, double(batch) * NO, loss, ctx->st);
-        }
+        launch_mlp_reduce(m, dweights, dbiases, loss ? sse : nullptr, ctx->st);
+        if (loss) launch_mlp_loss(sse, double(batch) * NO, loss, ctx->st);
         sync(ctx);
     });
 }
@@ -3389,7 +3377,6 @@ fjsph_status fjsph_surrogate_train(fjsph_ctx* ctx, int64_t n, const double* poin
         float* dT = tb.alloc<float>(T.size());
         int32_t* didx = tb.alloc<int32_t>(size_t(batch));
         float* p = tb.alloc<float>(size_t(np));
-        float* g = tb.alloc<float>(size_t(np));
         float* m1 = tb.alloc<float>(size_t(np));
         float* m2 = tb.alloc<float>(size_t(np));
         float* sse = tb.alloc<float>(size_t(std::max(steps, 1)));
@@ -3405,15 +3392,18 @@ fjsph_status fjsph_surrogate_train(fjsph_ctx* ctx, int64_t n, const double* poin
         m.X = dX;
         m.T = dT;
         m.idx = didx;
+        mlp_params(m, p, wf, wt);
         /* Adam (beta 0.9, 0.999, eps 1e-8) with a cosine learning-rate
          * schedule from lr to 0 over the steps */
         const double b1 = 0.9, b2 = 0.999;
         for (int32_t t = 1; t <= steps; ++t) {
-            launch_mlp_batch(seed, t, n, batch, didx, ctx->st);
-            mlp_pass(ctx, m, p, g, sse + (t - 1), wf, wt);
+            launch_mlp_pack_draw(D, p, L, wf, wt, seed, t, n, batch, didx, ctx->st);
+            launch_mlp_train(D, m, ctx->st);
             const double lr_t = lr * 0.5 * (1.0 + std::cos(3.14159265358979323846 * double(t - 1) / double(steps)));
-            launch_mlp_adam(p, g, m1, m2, np, float(lr_t), float(b1), float(b2), 1e-8f,
-                            float(1.0 - std::pow(b1, t)), float(1.0 - std::pow(b2, t)), ctx->st);
+            launch_mlp_reduce_adam(m, sse + (t - 1),
+                                   MlpAdam{p, m1, m2, float(lr_t), float(b1), float(b2), 1e-8f,
+                                           float(1.0 - std::pow(b1, t)), float(1.0 - std::pow(b2, t))},
+                                   ctx->st);
         }
         sync(ctx);
         HIPCHK(hipMemcpy(weights, p, size_t(m.nw) * 4, hipMemcpyDeviceToHost));

@@ -220,12 +220,17 @@ struct MlpTrain {
     const float* b;      /* hidden biases, n_hidden x 64                      */
     const float* bo;     /* output biases (D + 2)                             */
     float* Z;            /* pre-activations, n_hidden x batch x 64            */
-    __bf16* H;           /* activations (H_0 = input), (n_hidden + 1) x batch x 64 */
-    float* dWp;          /* per-wave weight-gradient partials, nw each        */
-    float* dbp;          /* per-wave bias-gradient partials, nb each          */
-    float* lossp;        /* per-wave sums of squared errors                   */
+    float* dWp;          /* per-block weight-gradient partials, nw each       */
+    float* dbp;          /* per-block bias-gradient partials, nb each         */
+    float* lossp;        /* per-block sums of squared errors                  */
     int64_t nw, nb;
     int32_t n_hidden, batch;
+};
+
+/* Adam's state (parameters p, moments m1, m2) and one step's constants. */
+struct MlpAdam {
+    float *p, *m1, *m2;
+    float lr, b1, b2, eps, c1, c2;
 };
 
 /* Scalars kept on the device between kernels. */
@@ -337,14 +342,18 @@ void launch_delete_flag(int dim, DevState s, const int32_t* part_id, const int32
                         int64_t n_bound, int32_t* keep, int32_t* hflag, int32_t* blkcount, hipStream_t st);
 void launch_compact_perm(const int32_t* keep, const int32_t* start, int64_t n, int32_t* perm, hipStream_t st);
 void launch_compact_ids(int32_t* part_id, const int32_t* hstart, int64_t n, hipStream_t st);
-void launch_mlp_batch(uint64_t seed, int64_t step, int64_t n, int32_t batch, int32_t* idx, hipStream_t st);
 void launch_mlp_train(int dim, const MlpTrain& m, hipStream_t st);
-void launch_mlp_reduce(const float* part, int64_t nwaves, int64_t stride, int64_t n, float* grad, hipStream_t st);
-void launch_mlp_adam(float* p, const float* g, float* m1, float* m2, int64_t n, float lr, float b1, float b2,
-                     float eps, float c1, float c2, hipStream_t st);
+/* Sums of the per-block partials: the gradients of the weights and biases,
+ * the squared error into *sse (null: not wanted). */
+void launch_mlp_reduce(const MlpTrain& m, float* gw, float* gb, float* sse, hipStream_t st);
+/* The same with the parameters updated by the gradients. */
+void launch_mlp_reduce_adam(const MlpTrain& m, float* sse, const MlpAdam& ad, hipStream_t st);
 int64_t mlp_tiles_fwd(int n_hidden);
 int64_t mlp_tiles_bwd(int n_hidden);
 void launch_mlp_pack(int dim, const float* w, int32_t n_hidden, void* wf, void* wt, hipStream_t st);
+/* The same, and the batch positions of step `step` drawn into idx. */
+void launch_mlp_pack_draw(int dim, const float* w, int32_t n_hidden, void* wf, void* wt, uint64_t seed, int64_t step,
+                          int64_t n, int32_t batch, int32_t* idx, hipStream_t st);
 /* Scratch of the entry points that allocate nothing (noalloc.hip): a
  * file-scope device array per GPU, its address taken once per device by
  * noalloc_init (with that device current) and returned by noalloc_scratch. */
