@@ -2028,6 +2028,15 @@ std::vector<int32_t>& slot_to_host(fjsph_ctx* ctx)
     return ctx->slot_host;
 }
 
+/* The host arrays are indexed by part_id: an inconsistent map (which
+ * launch_host_order found) must not reach them. */
+void check_host_order(fjsph_ctx* ctx)
+{
+    HIPCHK(hipMemcpyAsync(&ctx->sc_host->bad_id, &ctx->sc->bad_id, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->st));
+    sync(ctx);
+    if (ctx->sc_host->bad_id) throw std::string("internal: slot to host map out of range");
+}
+
 }  // namespace
 
 /* =========================================================== C entry points */
@@ -2774,18 +2783,11 @@ fjsph_status fjsph_download_field(fjsph_ctx* ctx, int32_t which, int32_t field, 
         require(ctx, false);
         DevState& st = which == FJSPH_STATE_N ? ctx->pn : ctx->pnp1;
         const int w = width_of(ctx, field);
-        const size_t cnt = size_t(ctx->n) * w;
-        std::vector<int32_t>& sh = slot_to_host(ctx);
-        if (field_desc(field).is_int) {
-            std::vector<int32_t> buf(cnt);
-            HIPCHK(hipMemcpy(buf.data(), *field_slot(st, field), cnt * 4, hipMemcpyDeviceToHost));
-            for (int64_t s = 0; s < ctx->n; ++s) out[sh[s]] = double(buf[s]);
-        } else {
-            std::vector<double> buf(cnt);
-            HIPCHK(hipMemcpy(buf.data(), *field_slot(st, field), cnt * 8, hipMemcpyDeviceToHost));
-            for (int64_t s = 0; s < ctx->n; ++s)
-                for (int k = 0; k < w; ++k) out[size_t(sh[s]) * w + k] = buf[size_t(s) * w + k];
-        }
+        double* dst = ctx->gather_tmp[field_desc(field).width_kind];
+        launch_host_order(*field_slot(st, field), field_desc(field).is_int, w, ctx->part_id, ctx->n, dst, ctx->sc,
+                          ctx->st);
+        check_host_order(ctx);
+        HIPCHK(hipMemcpy(out, dst, sizeof(double) * ctx->n * w, hipMemcpyDeviceToHost));
     });
 }
 

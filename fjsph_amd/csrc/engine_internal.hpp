@@ -250,6 +250,7 @@ struct DevScalars {
     int32_t fresh_n;   /* particles leaving the pipe listed for FirstCell */
     int32_t fc_count;  /* of those, in no cell (FirstCell's boundary branch) */
     int32_t fc_del;    /* of those, across a far-field face */
+    int32_t bad_id;    /* 1: a slot's host index out of range */
 };
 
 /* ---- launch wrappers (kernels.hip); every one enqueues on `st` ---------- */
@@ -275,6 +276,11 @@ void launch_export_lists(int dim, TileGrid tg, NbrList nl, int64_t n, int32_t* o
 void launch_aux(int dim, DevState s, Aux a, int64_t n, int ale, int mixed, double bgam, hipStream_t st);
 void launch_gather_d(const double* src, double* dst, const int32_t* perm, int64_t n, int width, hipStream_t st);
 void launch_gather_i(const int32_t* src, int32_t* dst, const int32_t* perm, int64_t n, hipStream_t st);
+/* dst[id[s]] = src[s] as FP64 (src int32 when is_int, else FP64), `width`
+ * values a slot; sc->bad_id is set to whether an id lies outside [0, n),
+ * whose slots are left out. */
+void launch_host_order(const void* src, bool is_int, int width, const int32_t* id, int64_t n, double* dst,
+                       DevScalars* sc, hipStream_t st);
 void launch_iota(int32_t* a, int64_t n, hipStream_t st);
 
 /* Pair passes.  r_from_x = 1 when the positions are those of the last
