@@ -1460,7 +1460,7 @@ __global__ __launch_bounds__(PTPB) void k_surface1_t(Consts c, DevState s, Aux a
     constexpr bool with_diss = MODE != 0;
     constexpr int TS = with_surf ? TILE : 1, TD = with_diss ? TILE : 1;
     __shared__ double tp[D][TILE], tv[D][TD], tg_[D][TD];
-    __shared__ double tvol[TILE], tlam[TS], trho[TD], tir[TD], tm[TD];
+    __shared__ double tvol[TILE], tlam[TS], trho[TD], tcs[TD], tm[TD];
     __shared__ int32_t tnb[TD], tsl[FR ? TILE : 1];
     __shared__ BlockHead h;
     block_head<D>(tg, h);
@@ -1529,7 +1529,7 @@ __global__ __launch_bounds__(PTPB) void k_surface1_t(Consts c, DevState s, Aux a
                         tg_[a][t] = s.gradRho[(int64_t)sl * D + a];
                     }
                     trho[t] = s.rho[sl];
-                    tir[t] = ax.invrho[sl];
+                    tcs[t] = sqrt(Bg * ax.invrho[sl]); /* sound speed: one root a slot, not one a pair */
                     tm[t] = s.m[sl];
                     tnb[t] = s.b[sl] > FJSPH_PISTON;
                 }
@@ -1576,7 +1576,7 @@ __global__ __launch_bounds__(PTPB) void k_surface1_t(Consts c, DevState s, Aux a
                         for (int a = 1; a < D; ++a) vdotr += Vji[a] * Rji[a];
                         if (!(vdotr > T(0))) {
                             const T muij = Ht * vdotr * idist2;
-                            const T cbar = T(0.5) * (cfac + fast_sqrt<T>(Bg * T(tir[t])));
+                            const T cbar = T(0.5) * (cfac + T(tcs[t]));
                             const T ff = T(tm[t]) * alpha * cbar * muij * fast_rcp<T>(T(0.5 * (rhoi + rhoj)));
 #pragma unroll
                             for (int a = 0; a < D; ++a) av[a] += double(g[a] * ff);
@@ -3204,15 +3204,19 @@ __device__ void skin_friction(const Consts& c, const double* Vd, const double* n
 #define FJ_FORCE_OCC __attribute__((amdgpu_waves_per_eu(4, 8)))
 #endif
 
-/* LDS tile of the FP64 force pass (parity path), one array per value: x, m,
- * v, p/rho^2, xb (FR), vPert, rho; 1/rho and m/rho are recomputed per pair
- * with the same operations as launch_aux, so they are bit-identical to the
- * stored ones. */
-template <bool FR>
+/* LDS tile of the FP64 force pass (parity path), one array per value.  1/rho
+ * and m/rho are launch_aux's: with the two divisions made again for every
+ * pair (the same operations, so the same bits) a pair was a chain of four,
+ * which the two waves per SIMD that the tile leaves room for do not hide,
+ * and without ALE the tile held zeros for vPert and rho.  200k-particle jet
+ * 0.95 -> 0.84 ms a launch, 4k droplet 0.248 -> 0.197, 345k particles in 2D
+ * 0.173 -> 0.132. */
+template <int D, bool FR, bool ALE>
 struct ForceTile {
-    double P[8][TILE];
-    double XB[3][FR ? TILE : 1];
-    double EA[4][TILE];
+    double X[D][TILE], V[D][TILE];
+    double m[TILE], P[TILE], ir[TILE], vol[TILE]; /* m negative for BOUND; p/rho^2 */
+    double XB[FR ? D : 1][FR ? TILE : 1];
+    double VP[ALE ? D : 1][ALE ? TILE : 1], rho[ALE ? TILE : 1];
 };
 
 /* Pair sums of get_acc_and_Rrho_on_i (src/Resid.cpp:243-418) for fluid
@@ -3222,12 +3226,12 @@ struct ForceTile {
  * surface-tension terms of a pair are combined before accumulation:
  * acc_i = sum_j (visc + ST / m_i - m_j (P_i + P_j) g).
  * FR: the positions have moved since the build, r comes from Aux::xb. */
-template <int D, bool FR>
-__global__ __launch_bounds__(PTPB) FJ_FORCE_OCC void k_force_t(Consts c, DevState s, Aux ax,
+template <int D, bool FR, bool ALE>
+__global__ __launch_bounds__(PTPB) void k_force_t(Consts c, DevState s, Aux ax,
                                                               const int32_t* __restrict__ part_id, TileGrid tg,
                                                               NbrList nl, const DevScalars* sc)
 {
-    __shared__ ForceTile<FR> ft;
+    __shared__ ForceTile<D, FR, ALE> ft;
     __shared__ BlockHead h;
     block_head<D>(tg, h);
     const int U = h.U;
@@ -3258,14 +3262,14 @@ __global__ __launch_bounds__(PTPB) FJ_FORCE_OCC void k_force_t(Consts c, DevStat
             xi[a] = active ? s.x[i * D + a] : 0.0;
             vi[a] = active ? s.v[i * D + a] : 0.0;
             xbi[a] = (FR && active) ? ax.xb[i * D + a] : 0.0;
-            vpi[a] = (fluid && c.ale) ? s.vPert[i * D + a] : 0.0;
+            vpi[a] = (fluid && ALE) ? s.vPert[i * D + a] : 0.0;
         }
         const double rhoi = fluid ? s.rho[i] : 1.0, mi = fluid ? s.m[i] : 1.0;
         const int32_t bi = fluid ? s.b[i] : 0;
         const double Pi = fluid ? ax.P[i] : 0.0;
         const double iri = fluid ? ax.invrho[i] : 0.0;
         const double inv_mi = 1.0 / mi;
-        const bool st_on = (!c.ale) || (fluid && s.surfzone[i] == 1);
+        const bool st_on = !ALE || (fluid && s.surfzone[i] == 1);
         const bool bound_i = bi == FJSPH_BOUND;
         double acc[D];
 #pragma unroll
@@ -3283,41 +3287,38 @@ __global__ __launch_bounds__(PTPB) FJ_FORCE_OCC void k_force_t(Consts c, DevStat
                 if (sl < 0) continue;
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
-                    ft.P[a][t] = s.x[(int64_t)sl * D + a];
-                    ft.P[4 + a][t] = s.v[(int64_t)sl * D + a];
-                    if constexpr (FR) ft.XB[FR ? a : 0][FR ? t : 0] = ax.xb[(int64_t)sl * D + a];
-                    ft.EA[a][t] = c.ale ? s.vPert[(int64_t)sl * D + a] : 0.0;
+                    ft.X[a][t] = s.x[(int64_t)sl * D + a];
+                    ft.V[a][t] = s.v[(int64_t)sl * D + a];
+                    if constexpr (FR) ft.XB[a][t] = ax.xb[(int64_t)sl * D + a];
+                    if constexpr (ALE) ft.VP[a][t] = s.vPert[(int64_t)sl * D + a];
                 }
-                ft.P[3][t] = s.b[sl] == FJSPH_BOUND ? -s.m[sl] : s.m[sl];
-                ft.P[7][t] = ax.P[sl];
-                ft.EA[3][t] = s.rho[sl];
+                ft.m[t] = s.b[sl] == FJSPH_BOUND ? -s.m[sl] : s.m[sl];
+                ft.P[t] = ax.P[sl];
+                ft.ir[t] = ax.invrho[sl];
+                ft.vol[t] = ax.vol[sl];
+                if constexpr (ALE) ft.rho[t] = s.rho[sl];
             }
             ts.load(tg, h, tk + 1, NT, U);
             __syncthreads();
             FJ_TILE_ENTRIES_BEGIN(cu, nl, base)
-                double Rji[D], Vji[D], vjr[D], vpj[D], xj[D], d2;
+                double Rji[D], Vji[D], vjr[D], xj[D], d2;
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
-                    xj[a] = ft.P[a][t];
+                    xj[a] = ft.X[a][t];
                     Rji[a] = xj[a] - xi[a];
-                    Vji[a] = ft.P[4 + a][t] - vi[a];
-                    vjr[a] = ft.P[4 + a][t];
-                    vpj[a] = ft.EA[a][t];
+                    vjr[a] = ft.V[a][t];
+                    Vji[a] = vjr[a] - vi[a];
                 }
                 if constexpr (FR) {
                     double xbj[D];
 #pragma unroll
-                    for (int a = 0; a < D; ++a) xbj[a] = ft.XB[FR ? a : 0][FR ? t : 0];
+                    for (int a = 0; a < D; ++a) xbj[a] = ft.XB[a][t];
                     d2 = exact_dist2<D>(xbi, xbj);
                 } else {
                     d2 = exact_dist2<D>(xi, xj);
                 }
                 const double rr = d2, r = sqrt(d2);
-                const double msg = ft.P[3][t];
-                const double Pj = ft.P[7][t];
-                const double rhoj = ft.EA[3][t];
-                const double irj = 1.0 / rhoj;
-                const double volj = fabs(msg) / rhoj;
+                const double msg = ft.m[t], Pj = ft.P[t], irj = ft.ir[t], volj = ft.vol[t];
                 const bool bound_j = msg < 0.0;
                 const double mj = bound_j ? -msg : msg;
                 const double idist2 = 1.0 / (rr + eps2);
@@ -3338,7 +3339,11 @@ __global__ __launch_bounds__(PTPB) FJ_FORCE_OCC void k_force_t(Consts c, DevStat
                 }
 #pragma unroll
                 for (int a = 0; a < D; ++a) acc[a] += vf * Vji[a] + sf * Rji[a] - pc * g[a];
-                if (c.ale) {
+                if constexpr (ALE) {
+                    const double rhoj = ft.rho[t];
+                    double vpj[D];
+#pragma unroll
+                    for (int a = 0; a < D; ++a) vpj[a] = ft.VP[a][t];
                     double aj = 0.0, ai = 0.0, cd = 0.0, cont = 0.0, c2 = 0.0;
 #pragma unroll
                     for (int a = 0; a < D; ++a) {
@@ -3360,15 +3365,19 @@ __global__ __launch_bounds__(PTPB) FJ_FORCE_OCC void k_force_t(Consts c, DevStat
                 }
             FJ_TILE_ENTRIES_END(cu, nl)
         }
-        split_fold(sp, acc, &ft.P[0][0], OpSum());
+        split_fold(sp, acc, &ft.X[0][0], OpSum());
         double rr2[2] = {Rrho_, Rrhoc_};
-        split_fold(sp, rr2, &ft.P[0][0], OpSum());
+        split_fold(sp, rr2, &ft.X[0][0], OpSum());
         Rrho_ = rr2[0];
         Rrhoc_ = rr2[1];
         if (!fluid || sp.part != 0) continue;
 #pragma unroll
         for (int a = 0; a < D; ++a) s.acc[i * D + a] = acc[a];
-        s.Rrho[i] = c.ale ? (Rrho_ * rhoi + Rrhoc_ + s.deltaD[i]) : (Rrho_ * rhoi + s.deltaD[i]);
+        {
+            /* rounded as written, whatever ALE makes of the code around it */
+#pragma clang fp contract(off)
+            s.Rrho[i] = (ALE ? fma(Rrho_, rhoi, Rrhoc_) : Rrho_ * rhoi) + s.deltaD[i];
+        }
     }
 }
 
@@ -3872,7 +3881,9 @@ void launch_force(int dim, const Consts& c, DevState s, Aux a, const int32_t* pa
                   int r_from_x, const DevScalars* sc, hipStream_t st)
 {
     const dim3 g((unsigned)tg.nblocks), b(PTPB);
-#define FJ_FORCE_T(DD, FF) hipLaunchKernelGGL((k_force_t<DD, FF>), g, b, 0, st, c, s, a, part_id, tg, nl, sc)
+#define FJ_FORCE_TA(DD, FF, AA) hipLaunchKernelGGL((k_force_t<DD, FF, AA>), g, b, 0, st, c, s, a, part_id, tg, nl, sc)
+#define FJ_FORCE_T(DD, FF) \
+    do { if (c.ale) FJ_FORCE_TA(DD, FF, true); else FJ_FORCE_TA(DD, FF, false); } while (0)
 #define FJ_FORCE_M(DD, FF, AA) hipLaunchKernelGGL((k_force_m<DD, FF, AA>), g, b, 0, st, c, s, a, part_id, tg, nl, sc)
 #define FJ_FORCE_MA(DD, FF) \
     do { if (c.ale) FJ_FORCE_M(DD, FF, true); else FJ_FORCE_M(DD, FF, false); } while (0)
@@ -3886,6 +3897,7 @@ void launch_force(int dim, const Consts& c, DevState s, Aux a, const int32_t* pa
 #undef FJ_FORCE_MA
 #undef FJ_FORCE_M
 #undef FJ_FORCE_T
+#undef FJ_FORCE_TA
 }
 
 void launch_nb_update(int dim, const Consts& c, DevState s, DevState pn, double* next_x, double* next_v,
