@@ -72,6 +72,32 @@ __device__ __forceinline__ void wendland(T r, T H, T inv_H, T Wc, T& W, T& fg)
     fg = (q < T(1e-12)) ? T(0) : T(5) * inv_H * inv_H * t3 * Wc;
 }
 
+/* Per-particle derived quantities of slot i (see Aux) from its density and
+ * pressure. */
+template <int D>
+__device__ __forceinline__ void aux_of(const DevState& s, const Aux& a, int64_t i, double rho, double p, int ale, int mixed,
+                                       float bgam)
+{
+    const double m = s.m[i];
+    const double vol = m / rho, P = p / (rho * rho), ir = 1.0 / rho;
+    a.vol[i] = vol;
+    a.P[i] = P;
+    a.invrho[i] = ir;
+    if (mixed) {
+        const int32_t b = s.b[i];
+        const float ms = b == FJSPH_BOUND ? -float(m) : float(m);
+        a.fq[i] = make_float4(ms, float(P), float(ir), float(vol));
+        a.fs2[i] = make_float4(float(vol), __builtin_amdgcn_sqrtf(bgam * float(ir)),
+                               b > FJSPH_PISTON ? float(m) : -float(m), 0.f);
+        if (ale) {
+            float vp[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < D; ++k) vp[k] = float(s.vPert[i * D + k]);
+            a.fale[i] = make_float4(vp[0], vp[1], vp[2], float(rho));
+        }
+    }
+}
+
 template <int D>
 __device__ __forceinline__ void load_vec(const double* __restrict__ a, int64_t i, double* out)
 {

@@ -173,7 +173,8 @@ struct fjsph_ctx {
     int32_t* export_buf = nullptr;
     bool x_at_build = false;   /* pnp1.x unchanged since the last build     */
     bool f64_tail = false;     /* this step's remaining force passes in FP64 */
-    int32_t* bnd_slots = nullptr; /* one boundary block's slots (count first), per pass */
+    int32_t* bnd_slots = nullptr; /* one boundary block's slots (count first) */
+    int32_t bnd_block = -1;       /* the block it lists, for the present order of the slots; -1: none */
     DevScalars* sc = nullptr;
     DevScalars* sc_host = nullptr; /* pinned */
     DevBlocks bl{};
@@ -543,12 +544,14 @@ void sync(fjsph_ctx* ctx) { HIPCHK(hipStreamSynchronize(ctx->st)); }
 
 void copy_state(fjsph_ctx* ctx, DevState& dst, DevState& src)
 {
+    static_assert(kNumFields <= CopyList::MAX, "a state's arrays go into one list");
+    CopyList cl;
     for (int f = 0; f < kNumFields; ++f) {
         void* d = *field_slot(dst, f);
         void* s = *field_slot(src, f);
-        const size_t bytes = size_t(ctx->n) * width_of(ctx, f) * (field_desc(f).is_int ? 4 : 8);
-        HIPCHK(hipMemcpyAsync(d, s, bytes, hipMemcpyDeviceToDevice, ctx->st));
+        cl.add(d, s, ctx->n * width_of(ctx, f) * (field_desc(f).is_int ? 4 : 8));
     }
+    launch_copy_list(cl, ctx->st);
 }
 
 /* Permute every per-slot array by perm (new slot s <- old slot perm[s]),
@@ -556,6 +559,7 @@ void copy_state(fjsph_ctx* ctx, DevState& dst, DevState& src)
 void permute_all(fjsph_ctx* ctx, const int32_t* perm, int64_t count = -1)
 {
     const int64_t n = count < 0 ? ctx->n : count;
+    ctx->bnd_block = -1;
     for (DevState* st : {&ctx->pn, &ctx->pnp1}) {
         for (int f = 0; f < kNumFields; ++f) {
             void** slot = field_slot(*st, f);
@@ -722,6 +726,7 @@ void block_shape(int dim, bool one_layer, bool f32, double cells, const int32_t 
 void build_neighbours(fjsph_ctx* ctx, bool reorder)
 {
     PassTimer t(ctx, FJSPH_T_NEIGHBOUR);
+    ctx->bnd_block = -1;
     const int D = ctx->s.dim;
     const int64_t n = ctx->n;
     const double cs = std::sqrt(ctx->d.sr) * (1.0 + 1e-7);
@@ -730,9 +735,7 @@ void build_neighbours(fjsph_ctx* ctx, bool reorder)
     if (grouped(ctx)) {
         ncell_d = group_layout(ctx, cs);
     } else {
-        launch_bbox(D, ctx->pnp1.x, n, ctx->partial, ctx->nparts, ctx->sc->bbox, ctx->st);
-        HIPCHK(hipMemcpyAsync(ctx->sc_host->bbox, ctx->sc->bbox, sizeof(double) * 6, hipMemcpyDeviceToHost,
-                              ctx->st));
+        launch_bbox(D, ctx->pnp1.x, n, ctx->partial, ctx->nparts, ctx->sc_host->bbox, ctx->st);
         sync(ctx);
         for (int k = 0; k < D; ++k) { lo[k] = ctx->sc_host->bbox[k]; hi[k] = ctx->sc_host->bbox[D + k]; }
         for (int k = 0; k < D; ++k)
@@ -761,8 +764,7 @@ void build_neighbours(fjsph_ctx* ctx, bool reorder)
     }
     ctx->ncell = ncell;
     const double inv_cs = 1.0 / cs;
-    HIPCHK(hipMemsetAsync(ctx->cell_count, 0, sizeof(int32_t) * ncell, ctx->st));
-    HIPCHK(hipMemsetAsync(ctx->cell_fill, 0, sizeof(int32_t) * ncell, ctx->st));
+    launch_clear_build(ctx->cell_count, ctx->cell_fill, ncell, ctx->sc, ctx->st);
     launch_cells(D, ctx->pnp1.x, n, lo, inv_cs, ctx->dims, ctx->cell, ctx->cell_count, ctx->st, ctx->grp, ctx->glo,
                  ctx->gl0);
     launch_scan(ctx->cell_count, ncell, ctx->cell_start, ctx->tile_sums, ctx->st);
@@ -808,7 +810,7 @@ void build_neighbours(fjsph_ctx* ctx, bool reorder)
     }
     set_tiles(bc);
     for (int attempt = 0; attempt < 40; ++attempt) {
-        HIPCHK(hipMemsetAsync(&ctx->sc->max_count, 0, 2 * sizeof(int32_t), ctx->st));
+        if (attempt > 0) HIPCHK(hipMemsetAsync(&ctx->sc->max_count, 0, 2 * sizeof(int32_t), ctx->st));
         launch_build_lists(D, ctx->pnp1.x, n, ctx->tg, ctx->d.sr, ctx->nl, ctx->sc, ctx->st);
         HIPCHK(hipMemcpyAsync(&ctx->sc_host->max_count, &ctx->sc->max_count, 2 * sizeof(int32_t),
                               hipMemcpyDeviceToHost, ctx->st));
@@ -1161,13 +1163,16 @@ void boundary_update(fjsph_ctx* ctx)
     for (size_t k = 0; k < ctx->blocks.size(); ++k) {
         if (ctx->blocks[k].b.is_fluid) continue;
         launch_boundary(ctx->s.dim, ctx->c, ctx->pnp1, ctx->aux, ctx->blk, ctx->bl, int32_t(k), ctx->tg, ctx->nl,
-                        ctx->n, ctx->nb, ctx->bnd_slots, ctx->near_inlet, ctx->st);
+                        ctx->n, ctx->nb, ctx->bnd_slots, ctx->bnd_block == int32_t(k), ctx->near_inlet, ctx->st);
+        ctx->bnd_block = int32_t(k);
     }
 }
 
-void force(fjsph_ctx* ctx, bool update)
+/* aux_fresh: boundary_update ran just before, whose solvers keep Aux up to
+ * date. */
+void force(fjsph_ctx* ctx, bool update, bool aux_fresh = false)
 {
-    refresh_aux(ctx);
+    if (!aux_fresh) refresh_aux(ctx);
     {
         PassTimer t(ctx, FJSPH_T_FORCE);
         NbrList nl64 = ctx->nl;
@@ -1214,7 +1219,7 @@ void force(fjsph_ctx* ctx, bool update)
 double nb_iter(fjsph_ctx* ctx)
 {
     boundary_update(ctx);
-    force(ctx, true);
+    force(ctx, true, ctx->nb > 0);
     std::swap(ctx->pnp1.x, ctx->x_nxt);
     std::swap(ctx->pnp1.v, ctx->v_nxt);
     std::swap(ctx->pnp1.rho, ctx->rho_nxt);
@@ -1223,9 +1228,7 @@ double nb_iter(fjsph_ctx* ctx)
     {
         PassTimer t(ctx, FJSPH_T_REDUCE);
         /* one residual partial per TPB slots (k_nb_update) */
-        launch_sum_partials(ctx->partial, reduction_parts(ctx->n), 1, &ctx->sc->residual, ctx->st);
-        HIPCHK(hipMemcpyAsync(&ctx->sc_host->residual, &ctx->sc->residual, sizeof(double), hipMemcpyDeviceToHost,
-                              ctx->st));
+        launch_sum_partials(ctx->partial, reduction_parts(ctx->n), 1, &ctx->sc_host->residual, ctx->st);
     }
     sync(ctx);
     const double nf = double(ctx->n - ctx->nb);
@@ -1269,8 +1272,7 @@ double find_timestep(fjsph_ctx* ctx)
     {
         PassTimer t(ctx, FJSPH_T_REDUCE);
         launch_timestep_reduce(ctx->s.dim, ctx->c, ctx->pnp1, ctx->part_id, ctx->n, ctx->partial, ctx->nparts,
-                               ctx->sc->red, ctx->st);
-        HIPCHK(hipMemcpyAsync(ctx->sc_host->red, ctx->sc->red, sizeof(double) * 7, hipMemcpyDeviceToHost, ctx->st));
+                               ctx->sc_host->red, ctx->st);
     }
     sync(ctx);
     return timestep_of(ctx, *ctx, ctx->sc_host->red, ctx->current_time, ctx->last_frame_time);
@@ -1383,7 +1385,7 @@ void upload_group_dt(fjsph_ctx* ctx)
 void nb_iter_groups(fjsph_ctx* ctx, std::vector<double>& le)
 {
     boundary_update(ctx);
-    force(ctx, true);
+    force(ctx, true, ctx->nb > 0);
     std::swap(ctx->pnp1.x, ctx->x_nxt);
     std::swap(ctx->pnp1.v, ctx->v_nxt);
     std::swap(ctx->pnp1.rho, ctx->rho_nxt);
@@ -1424,8 +1426,7 @@ void rebuild_groups(fjsph_ctx* ctx, const std::vector<int32_t>& mask)
             }
         const double cs = std::sqrt(ctx->d.sr) * (1.0 + 1e-7);
         const double lo[3] = {0, 0, 0};
-        HIPCHK(hipMemsetAsync(ctx->cell_count, 0, sizeof(int32_t) * ctx->ncell, ctx->st));
-        HIPCHK(hipMemsetAsync(ctx->cell_fill, 0, sizeof(int32_t) * ctx->ncell, ctx->st));
+        launch_clear_build(ctx->cell_count, ctx->cell_fill, ctx->ncell, ctx->sc, ctx->st);
         launch_cells(D, ctx->aux.xb, n, lo, 1.0 / cs, ctx->dims, ctx->cell, ctx->cell_count, ctx->st, ctx->grp,
                      ctx->glo, ctx->gl0);
         launch_scan(ctx->cell_count, ctx->ncell, ctx->cell_start, ctx->tile_sums, ctx->st);
@@ -1433,7 +1434,6 @@ void rebuild_groups(fjsph_ctx* ctx, const std::vector<int32_t>& mask)
         launch_sort_cells(ctx->cell_start, ctx->ncell, ctx->order, ctx->st);
         HIPCHK(hipMemcpyAsync(ctx->gbuild, mask.data(), sizeof(int32_t) * mask.size(), hipMemcpyHostToDevice,
                               ctx->st));
-        HIPCHK(hipMemsetAsync(&ctx->sc->max_count, 0, 2 * sizeof(int32_t), ctx->st));
         TileGrid tg = ctx->tg;
         tg.gbuild = ctx->gbuild;
         launch_build_lists(D, ctx->aux.xb, n, tg, ctx->d.sr, ctx->nl, ctx->sc, ctx->st);
@@ -1564,7 +1564,8 @@ void rk_stage(fjsph_ctx* ctx, DevState& dst, DevState& prev, double dt, bool fin
         for (size_t k = 0; k < ctx->blocks.size(); ++k) {
             if (ctx->blocks[k].b.is_fluid) continue;
             launch_boundary(D, ctx->c, dst, ctx->aux, ctx->blk, ctx->bl, int32_t(k), ctx->tg, ctx->nl, ctx->n,
-                            ctx->nb, ctx->bnd_slots, ctx->near_inlet, ctx->st);
+                            ctx->nb, ctx->bnd_slots, ctx->bnd_block == int32_t(k), ctx->near_inlet, ctx->st);
+            ctx->bnd_block = int32_t(k);
         }
         launch_rk_bnd_rho(D, ctx->c, dst, ctx->pn, ctx->rk1, ctx->rk2, ctx->rk3, ctx->blk, ctx->bl, ctx->near_inlet,
                           ctx->n, dt, final_stage ? 1 : 0, ctx->st);
@@ -1593,9 +1594,7 @@ double rk_error(fjsph_ctx* ctx, const DevState& a, const DevState& b, double log
     {
         PassTimer t(ctx, FJSPH_T_REDUCE);
         launch_sqdiff(ctx->s.dim, a.x, b.x, ctx->part_id, ctx->nb, ctx->n, ctx->partial, ctx->st);
-        launch_sum_partials(ctx->partial, reduction_parts(ctx->n), 1, &ctx->sc->residual, ctx->st);
-        HIPCHK(hipMemcpyAsync(&ctx->sc_host->residual, &ctx->sc->residual, sizeof(double), hipMemcpyDeviceToHost,
-                              ctx->st));
+        launch_sum_partials(ctx->partial, reduction_parts(ctx->n), 1, &ctx->sc_host->residual, ctx->st);
     }
     sync(ctx);
     const double nf = double(ctx->n - ctx->nb);
@@ -2148,6 +2147,7 @@ fjsph_status fjsph_upload_state(fjsph_ctx* ctx, int64_t n_total, int64_t n_bound
         HIPCHK(hipMemcpy(ctx->part_id, ids.data(), sizeof(int32_t) * n_total, hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(ctx->pn.pid, ids.data(), sizeof(int32_t) * n_total, hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(ctx->pnp1.pid, ids.data(), sizeof(int32_t) * n_total, hipMemcpyHostToDevice));
+        ctx->bnd_block = -1;
         HIPCHK(hipMemcpy(ctx->blk, blk.data(), sizeof(int32_t) * n_total, hipMemcpyHostToDevice));
         ctx->c.n_bound = n_bound;
         ctx->have_state = true;
@@ -2212,6 +2212,7 @@ fjsph_status fjsph_set_blocks(fjsph_ctx* ctx, int32_t n_blocks, const fjsph_bloc
             for (int k = 0; k < n_blocks; ++k)
                 if (h >= blocks[k].first && h < blocks[k].last) { blk[s] = k; break; }
         }
+        ctx->bnd_block = -1;
         HIPCHK(hipMemcpy(ctx->blk, blk.data(), sizeof(int32_t) * ctx->n, hipMemcpyHostToDevice));
         const int nbk = n_blocks;
         std::vector<int32_t> solver(std::max(nbk, 1)), ns(std::max(nbk, 1));

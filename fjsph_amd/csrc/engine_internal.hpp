@@ -236,7 +236,8 @@ struct MlpAdam {
 /* Scalars kept on the device between kernels. */
 struct DevScalars {
     double npd;       /* numerical particle density of the last dSPH pass */
-    double residual;  /* sum |x' - x_prev|^2 of the last Newmark iterate */
+    double residual;  /* sum |x' - x_prev|^2 of the last Newmark iterate; this, red and bbox are written
+                         to the pinned host copy by the kernels themselves */
     double red[8];    /* find_timestep reduction results */
     double bbox[6];   /* lo[3], hi[3] */
     int32_t max_count;
@@ -276,6 +277,19 @@ void launch_export_lists(int dim, TileGrid tg, NbrList nl, int64_t n, int32_t* o
 void launch_aux(int dim, DevState s, Aux a, int64_t n, int ale, int mixed, double bgam, hipStream_t st);
 void launch_gather_d(const double* src, double* dst, const int32_t* perm, int64_t n, int width, hipStream_t st);
 void launch_gather_i(const int32_t* src, int32_t* dst, const int32_t* perm, int64_t n, hipStream_t st);
+/* Arrays to copy together: at most MAX, whole multiples of 4 B, from and to
+ * addresses of 16 B. */
+struct CopyList {
+    static constexpr int MAX = 48;
+    void* dst[MAX];
+    const void* src[MAX];
+    int64_t bytes[MAX];
+    int32_t first[MAX + 1] = {0}; /* first block of each array */
+    int32_t n = 0;
+    void add(void* d, const void* s, int64_t b);
+};
+void launch_copy_list(const CopyList& cl, hipStream_t st);
+void launch_clear_build(int32_t* count, int32_t* fill, int64_t ncell, DevScalars* sc, hipStream_t st);
 /* dst[id[s]] = src[s] as FP64 (src int32 when is_int, else FP64), `width`
  * values a slot; sc->bad_id is set to whether an id lies outside [0, n),
  * whose slots are left out. */
@@ -300,7 +314,7 @@ void launch_shift(int dim, const Consts& c, DevState s, Aux a, const int32_t* pa
 void launch_surface2_shift(int dim, const Consts& c, DevState s, Aux a, const int32_t* part_id, TileGrid tg,
                            NbrList nl, int64_t n, int r_from_x, const double* norms_tmp, hipStream_t st);
 void launch_boundary(int dim, const Consts& c, DevState s, Aux a, const int32_t* blk, DevBlocks bl, int32_t block,
-                     TileGrid tg, NbrList nl, int64_t n, int64_t nb, int32_t* slots, int32_t* near_inlet,
+                     TileGrid tg, NbrList nl, int64_t n, int64_t nb, int32_t* slots, bool listed, int32_t* near_inlet,
                      hipStream_t st);
 /* Force pass on `s`; when next_x is non-null the Newmark update of
  * Do_NB_Iter is fused and writes next x/v/rho/p for every slot, plus one

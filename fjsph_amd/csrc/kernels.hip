@@ -299,30 +299,11 @@ void launch_sort_cells(const int32_t* start, int64_t ncell, int32_t* order, hipS
     hipLaunchKernelGGL(k_sort_cells, dim3((unsigned)g), dim3(64), 0, st, start, ncell, order);
 }
 
-/* Per-particle derived quantities (see Aux). */
 template <int D>
 __global__ __launch_bounds__(TPB) void k_aux(DevState s, Aux a, int64_t n, int ale, int mixed, float bgam)
 {
     const int64_t i = blockIdx.x * (int64_t)TPB + threadIdx.x;
-    if (i >= n) return;
-    const double rho = s.rho[i], m = s.m[i], p = s.p[i];
-    const double vol = m / rho, P = p / (rho * rho), ir = 1.0 / rho;
-    a.vol[i] = vol;
-    a.P[i] = P;
-    a.invrho[i] = ir;
-    if (mixed) {
-        const int32_t b = s.b[i];
-        const float ms = b == FJSPH_BOUND ? -float(m) : float(m);
-        a.fq[i] = make_float4(ms, float(P), float(ir), float(vol));
-        a.fs2[i] = make_float4(float(vol), __builtin_amdgcn_sqrtf(bgam * float(ir)),
-                               b > FJSPH_PISTON ? float(m) : -float(m), 0.f);
-        if (ale) {
-            float vp[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-            for (int k = 0; k < D; ++k) vp[k] = float(s.vPert[i * D + k]);
-            a.fale[i] = make_float4(vp[0], vp[1], vp[2], float(rho));
-        }
-    }
+    if (i < n) aux_of<D>(s, a, i, s.rho[i], s.p[i], ale, mixed, bgam);
 }
 
 void launch_aux(int dim, DevState s, Aux a, int64_t n, int ale, int mixed, double bgam, hipStream_t st)
@@ -398,6 +379,61 @@ void launch_host_order(const void* src, bool is_int, int width, const int32_t* i
     hipLaunchKernelGGL(k_clear_bad_id, dim3(1), dim3(1), 0, st, sc);
     if (is_int) hipLaunchKernelGGL(k_host_order<int32_t>, g, b, 0, st, (const int32_t*)src, dst, id, n, width, sc);
     else hipLaunchKernelGGL(k_host_order<double>, g, b, 0, st, (const double*)src, dst, id, n, width, sc);
+}
+
+/* Every array of a list copied by one launch, 16 KB to a block.  A state is
+ * 33 arrays; as copies of their own they took 4 us each whatever their size
+ * (0.13 ms a state, and a Runge-Kutta step copies six). */
+constexpr int64_t COPY_BYTES = TPB * 4 * 16;
+
+__global__ __launch_bounds__(TPB) void k_copy_list(CopyList cl)
+{
+    int k = 0;
+    for (int step = 32; step > 0; step >>= 1)
+        if (k + step < cl.n && int(blockIdx.x) >= cl.first[k + step]) k += step;
+    const int64_t at = int64_t(int(blockIdx.x) - cl.first[k]) * COPY_BYTES;
+    const char* src = (const char*)cl.src[k] + at;
+    char* dst = (char*)cl.dst[k] + at;
+    const int64_t left = cl.bytes[k] - at;
+    if (left >= COPY_BYTES) {
+        int4 v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = ((const int4*)src)[r * TPB + threadIdx.x];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ((int4*)dst)[r * TPB + threadIdx.x] = v[r];
+    } else {
+        for (int64_t w = threadIdx.x; w < left / 4; w += TPB) ((int32_t*)dst)[w] = ((const int32_t*)src)[w];
+    }
+}
+
+void CopyList::add(void* d, const void* s, int64_t b)
+{
+    if (b <= 0) return;
+    dst[n] = d;
+    src[n] = s;
+    bytes[n] = b;
+    first[n + 1] = first[n] + int32_t((b + COPY_BYTES - 1) / COPY_BYTES);
+    ++n;
+}
+
+void launch_copy_list(const CopyList& cl, hipStream_t st)
+{
+    if (cl.n > 0) hipLaunchKernelGGL(k_copy_list, dim3((unsigned)cl.first[cl.n]), dim3(TPB), 0, st, cl);
+}
+
+/* The cell counters and the list build's counters, before a build. */
+__global__ __launch_bounds__(TPB) void k_clear_build(int32_t* count, int32_t* fill, int64_t ncell, DevScalars* sc)
+{
+    const int64_t i = blockIdx.x * (int64_t)TPB + threadIdx.x;
+    if (i == 0) sc->max_count = sc->overflow = 0;
+    if (i >= ncell) return;
+    count[i] = 0;
+    fill[i] = 0;
+}
+
+void launch_clear_build(int32_t* count, int32_t* fill, int64_t ncell, DevScalars* sc, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_clear_build, dim3(grid_of(ncell)), dim3(TPB), 0, st, count, fill, ncell, sc);
 }
 
 /* Sum `width` columns of per-block partials in a fixed order, times scale. */

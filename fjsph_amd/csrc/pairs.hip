@@ -2997,8 +2997,11 @@ __global__ __launch_bounds__(TPB) void k_bnd_solve(Consts c, DevState s, Aux ax,
             pres = near ? fmax(0.0, pp) : pp;
         }
         if (lead) {
+            const double rho = eos_density(c, pres);
             s.p[i] = pres;
-            s.rho[i] = eos_density(c, pres);
+            s.rho[i] = rho;
+            /* what the force pass reads of the particle, as of now */
+            aux_of<D>(s, ax, i, rho, pres, c.ale, nl.f32, float(c.B * c.gam));
         }
     } else if (solver == FJSPH_GHOST) {
         int ni = 1;
@@ -3025,12 +3028,17 @@ __global__ __launch_bounds__(TPB) void k_bnd_solve(Consts c, DevState s, Aux ax,
 }
 
 void launch_boundary(int dim, const Consts& c, DevState s, Aux a, const int32_t* blk, DevBlocks bl, int32_t block,
-                     TileGrid tg, NbrList nl, int64_t n, int64_t nb, int32_t* slots, int32_t* near_inlet,
+                     TileGrid tg, NbrList nl, int64_t n, int64_t nb, int32_t* slots, bool listed, int32_t* near_inlet,
                      hipStream_t st)
 {
-    /* the block's slots (at most nb, the boundary count), then one wave each */
-    hipLaunchKernelGGL(k_clear_count, dim3(1), dim3(1), 0, st, slots);
-    hipLaunchKernelGGL(k_block_slots, dim3(grid_of(n)), dim3(TPB), 0, st, blk, n, block, slots);
+    /* the block's slots (at most nb, the boundary count), listed once for an
+     * order of the slots, then one wave each: with Aux kept up by k_bnd_solve
+     * a sub-iteration has three launches of 5-8 us fewer (6.5k particles 1.17
+     * -> 1.02 ms a step, of which the FP64 dSPH pass 0.01) */
+    if (!listed) {
+        hipLaunchKernelGGL(k_clear_count, dim3(1), dim3(1), 0, st, slots);
+        hipLaunchKernelGGL(k_block_slots, dim3(grid_of(n)), dim3(TPB), 0, st, blk, n, block, slots);
+    }
     const dim3 g((unsigned)((nb + TPB / 64 - 1) / (TPB / 64))), b(TPB);
     if (dim == 2) {
         hipLaunchKernelGGL(k_bnd_vel<2>, g, b, 0, st, c, s, a, bl, block, tg, nl, slots);

@@ -3,7 +3,7 @@ made of the order on the device."""
 import numpy as np
 import pytest
 
-from fjsph_amd import abi
+from fjsph_amd import abi, cases
 from tests.test_gpu_parity import _engine, _small_cases
 
 pytestmark = pytest.mark.gpu
@@ -25,4 +25,22 @@ def test_host_order(name, which):
                  ("L", k[:, None] + np.arange(dim * dim) / 16)):
         eng.set_field(f, v, which)
         assert np.array_equal(eng.field(f, which), v), f
+    eng.close()
+
+
+@pytest.mark.parametrize("n", [64, 1023, 2048, 2049, 4097])
+def test_state_copy(n):
+    """The step's end copies one state over the other in one launch: sizes
+    around the launch's blocks of 16 KB (2048 scalars, 4096 integers), odd
+    ones with a remainder of 4 and 8 B."""
+    case = cases.fluid_block(3, 17, dx=1e-3, precision=abi.PREC_FP64, H_fac=2.0, sig=0.07)
+    for f in ("x", "v", "rho", "p", "m", "b"):
+        setattr(case, f, np.ascontiguousarray(getattr(case, f)[:n]))
+    case.blocks = [dict(first=0, last=n, is_fluid=1)]
+    print(f"[fields] state copy n={n}", flush=True)
+    eng = _engine(case)
+    eng.integrate_no_update()
+    eng.integrate_step()
+    for f in abi.F:
+        assert np.array_equal(eng.field(f, abi.STATE_N), eng.field(f, abi.STATE_NP1)), f
     eng.close()
