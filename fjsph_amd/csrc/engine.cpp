@@ -159,6 +159,9 @@ struct fjsph_ctx {
     int nparts = 0;
     double* gather_tmp[3] = {nullptr, nullptr, nullptr}; /* spare field buffers: scalar, vector, matrix */
     int32_t* gather_tmp_i = nullptr;
+    DevState spare{};               /* small sets: buffers for a whole state's permutation at once */
+    int32_t* spare_i[6] = {nullptr}; /* and for the further per-slot arrays */
+    int64_t spare_cap = 0;           /* slots they hold (0: none) */
 
     /* cell grid */
     int32_t *cell = nullptr, *cell_count = nullptr, *cell_start = nullptr, *cell_fill = nullptr;
@@ -313,8 +316,16 @@ void free_state(DevState& s)
     }
 }
 
+void free_spare(fjsph_ctx* ctx)
+{
+    free_state(ctx->spare);
+    for (int32_t*& a : ctx->spare_i) dfree(a);
+    ctx->spare_cap = 0;
+}
+
 void free_all(fjsph_ctx* ctx)
 {
+    free_spare(ctx);
     free_state(ctx->pn);
     free_state(ctx->pnp1);
     free_state(ctx->rk1);
@@ -554,12 +565,58 @@ void copy_state(fjsph_ctx* ctx, DevState& dst, DevState& src)
     launch_copy_list(cl, ctx->st);
 }
 
+/* Buffers for all arrays of a state at once, of the states' own capacity
+ * (they change places with the state's); false where there is no room. */
+bool have_spare(fjsph_ctx* ctx)
+{
+    const int64_t cap = std::max(ctx->cap, ctx->n);
+    if (ctx->spare_cap == cap) return true;
+    free_spare(ctx);
+    try {
+        for (int f = 0; f < kNumFields; ++f) {
+            void** slot = field_slot(ctx->spare, f);
+            const size_t cnt = size_t(cap) * width_of(ctx, f);
+            if (field_desc(f).is_int) dalloc(*(int32_t**)slot, cnt);
+            else dalloc(*(double**)slot, cnt);
+        }
+        for (int32_t*& a : ctx->spare_i) dalloc(a, size_t(cap));
+    } catch (const HipError&) {
+        (void)hipGetLastError();
+        free_spare(ctx);
+        return false;
+    }
+    ctx->spare_cap = cap;
+    return true;
+}
+
 /* Permute every per-slot array by perm (new slot s <- old slot perm[s]),
- * for the first `count` new slots (ctx->n when negative). */
+ * for the first `count` new slots (ctx->n when negative).  Up to
+ * kGatherTogether slots a gather is shorter than its launch (2.4 us of 5),
+ * and all arrays of a state go in one, into a second set of buffers; above
+ * it, array by array into one spare buffer of each width (8 us a gather at
+ * 700k), without a state's worth of memory. */
+constexpr int64_t kGatherTogether = 300000;
+
 void permute_all(fjsph_ctx* ctx, const int32_t* perm, int64_t count = -1)
 {
     const int64_t n = count < 0 ? ctx->n : count;
     ctx->bnd_block = -1;
+    int32_t** const more[6] = {&ctx->part_id, &ctx->blk, &ctx->cell, &ctx->col, &ctx->depth, &ctx->grp};
+    if (n > 0 && ctx->n <= kGatherTogether && have_spare(ctx)) {
+        for (DevState* st : {&ctx->pn, &ctx->pnp1}) {
+            GatherList gl;
+            for (int f = 0; f < kNumFields; ++f)
+                gl.add(*field_slot(ctx->spare, f), *field_slot(*st, f), width_of(ctx, f), field_desc(f).is_int, n);
+            if (st == &ctx->pn)
+                for (int k = 0; k < 6; ++k)
+                    if (*more[k]) gl.add(ctx->spare_i[k], *more[k], 1, true, n);
+            launch_gather_list(gl, perm, n, ctx->st);
+            std::swap(*st, ctx->spare);
+        }
+        for (int k = 0; k < 6; ++k)
+            if (*more[k]) std::swap(*more[k], ctx->spare_i[k]);
+        return;
+    }
     for (DevState* st : {&ctx->pn, &ctx->pnp1}) {
         for (int f = 0; f < kNumFields; ++f) {
             void** slot = field_slot(*st, f);
@@ -576,7 +633,7 @@ void permute_all(fjsph_ctx* ctx, const int32_t* perm, int64_t count = -1)
             }
         }
     }
-    for (int32_t** arr : {&ctx->part_id, &ctx->blk, &ctx->cell, &ctx->col, &ctx->depth, &ctx->grp}) {
+    for (int32_t** arr : more) {
         if (!*arr) continue;
         launch_gather_i(*arr, ctx->gather_tmp_i, perm, n, ctx->st);
         std::swap(*arr, ctx->gather_tmp_i);

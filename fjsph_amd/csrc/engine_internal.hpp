@@ -289,6 +289,18 @@ struct CopyList {
     void add(void* d, const void* s, int64_t b);
 };
 void launch_copy_list(const CopyList& cl, hipStream_t st);
+/* Arrays to gather together by one permutation: `width` values a slot, FP64
+ * or int32. */
+struct GatherList {
+    static constexpr int MAX = 48;
+    void* dst[MAX];
+    const void* src[MAX];
+    int32_t width[MAX]; /* negative: int32 */
+    int32_t first[MAX + 1] = {0};
+    int32_t n = 0;
+    void add(void* d, const void* s, int w, bool is_int, int64_t slots);
+};
+void launch_gather_list(const GatherList& gl, const int32_t* perm, int64_t n, hipStream_t st);
 void launch_clear_build(int32_t* count, int32_t* fill, int64_t ncell, DevScalars* sc, hipStream_t st);
 /* dst[id[s]] = src[s] as FP64 (src int32 when is_int, else FP64), `width`
  * values a slot; sc->bad_id is set to whether an id lies outside [0, n),

@@ -145,8 +145,10 @@ void launch_cells(int dim, const double* x, int64_t n, const double* lo, double 
     else hipLaunchKernelGGL(k_cells<3>, dim3(grid_of(n)), dim3(TPB), 0, st, x, n, g, cell, cell_count);
 }
 
-/* Three-phase exclusive scan over tiles of SCAN_TILE counts. */
-constexpr int SCAN_TILE = 2048;
+/* Exclusive scan over tiles of SCAN_TILE counts: the tiles' sums, then the
+ * tiles, each adding up the sums before it (up to SCAN_DIRECT tiles, four
+ * loads a thread; above, the sums are scanned by a launch between). */
+constexpr int SCAN_TILE = 2048, SCAN_DIRECT = 1024;
 
 __device__ int32_t block_excl_scan_i(int32_t v, int32_t* lds, int32_t& total)
 {
@@ -199,11 +201,19 @@ __global__ __launch_bounds__(TPB) void k_scan_sums(int32_t* tile_sums, int ntile
 }
 
 __global__ __launch_bounds__(TPB) void k_scan_apply(const int32_t* __restrict__ count, int64_t ncell,
-                                                    const int32_t* __restrict__ tile_sums, int32_t* start)
+                                                    const int32_t* __restrict__ tile_sums, int scanned, int32_t* start)
 {
     __shared__ int32_t lds[NWAVE];
     constexpr int PER = SCAN_TILE / TPB;
     const int64_t base = blockIdx.x * (int64_t)SCAN_TILE + threadIdx.x * PER;
+    int32_t before = 0;
+    if (scanned) {
+        before = tile_sums[blockIdx.x];
+    } else if (blockIdx.x > 0) {
+        int32_t mine = 0;
+        for (int t = threadIdx.x; t < int(blockIdx.x); t += TPB) mine += tile_sums[t];
+        (void)block_excl_scan_i(mine, lds, before);
+    }
     int32_t v[PER];
     int32_t s = 0;
 #pragma unroll
@@ -212,26 +222,22 @@ __global__ __launch_bounds__(TPB) void k_scan_apply(const int32_t* __restrict__ 
         s += v[k];
     }
     int32_t total;
-    int32_t ex = block_excl_scan_i(s, lds, total) + tile_sums[blockIdx.x];
+    int32_t ex = block_excl_scan_i(s, lds, total) + before;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
         if (base + k < ncell) start[base + k] = ex;
         ex += v[k];
     }
-}
-
-__global__ void k_scan_total(const int32_t* count, int64_t ncell, int32_t* start)
-{
-    start[ncell] = start[ncell - 1] + count[ncell - 1];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) start[ncell] = before + total;
 }
 
 void launch_scan(const int32_t* count, int64_t ncell, int32_t* start, int32_t* tile_sums, hipStream_t st)
 {
     const int ntiles = (int)((ncell + SCAN_TILE - 1) / SCAN_TILE);
-    hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(TPB), 0, st, count, ncell, tile_sums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(TPB), 0, st, tile_sums, ntiles);
-    hipLaunchKernelGGL(k_scan_apply, dim3(ntiles), dim3(TPB), 0, st, count, ncell, tile_sums, start);
-    hipLaunchKernelGGL(k_scan_total, dim3(1), dim3(1), 0, st, count, ncell, start);
+    const int scanned = ntiles > SCAN_DIRECT;
+    if (ntiles > 1) hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(TPB), 0, st, count, ncell, tile_sums);
+    if (scanned) hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(TPB), 0, st, tile_sums, ntiles);
+    hipLaunchKernelGGL(k_scan_apply, dim3(ntiles), dim3(TPB), 0, st, count, ncell, tile_sums, scanned, start);
 }
 
 __global__ __launch_bounds__(TPB) void k_scatter(const int32_t* __restrict__ cell, int64_t n,
@@ -419,6 +425,43 @@ void CopyList::add(void* d, const void* s, int64_t b)
 void launch_copy_list(const CopyList& cl, hipStream_t st)
 {
     if (cl.n > 0) hipLaunchKernelGGL(k_copy_list, dim3((unsigned)cl.first[cl.n]), dim3(TPB), 0, st, cl);
+}
+
+/* Every array of a list gathered by one launch, 4 values to a thread. */
+constexpr int GATHER_VALUES = TPB * 4;
+
+__global__ __launch_bounds__(TPB) void k_gather_list(GatherList gl, const int32_t* __restrict__ perm, int32_t n)
+{
+    int k = 0;
+    for (int step = 32; step > 0; step >>= 1)
+        if (k + step < gl.n && int(blockIdx.x) >= gl.first[k + step]) k += step;
+    const uint32_t t0 = uint32_t(int(blockIdx.x) - gl.first[k]) * GATHER_VALUES + threadIdx.x;
+    const uint32_t w = uint32_t(abs(gl.width[k])), total = uint32_t(n) * w;
+    const bool is_int = gl.width[k] < 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const uint32_t t = t0 + r * TPB;
+        if (t >= total) return;
+        const uint32_t s = t / w;
+        const int64_t from = int64_t(perm[s]) * w + (t - s * w);
+        if (is_int) ((int32_t*)gl.dst[k])[t] = ((const int32_t*)gl.src[k])[from];
+        else ((double*)gl.dst[k])[t] = ((const double*)gl.src[k])[from];
+    }
+}
+
+void GatherList::add(void* d, const void* s, int w, bool is_int, int64_t slots)
+{
+    dst[n] = d;
+    src[n] = s;
+    width[n] = is_int ? -w : w;
+    first[n + 1] = first[n] + int32_t((slots * w + GATHER_VALUES - 1) / GATHER_VALUES);
+    ++n;
+}
+
+void launch_gather_list(const GatherList& gl, const int32_t* perm, int64_t n, hipStream_t st)
+{
+    if (gl.n > 0 && n > 0)
+        hipLaunchKernelGGL(k_gather_list, dim3((unsigned)gl.first[gl.n]), dim3(TPB), 0, st, gl, perm, int32_t(n));
 }
 
 /* The cell counters and the list build's counters, before a build. */

@@ -10,9 +10,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("which", [abi.STATE_NP1, abi.STATE_N], ids=["np1", "n"])
-@pytest.mark.parametrize("name", ["drop3d", "dam2d"])
+@pytest.mark.parametrize("name", ["drop3d", "dam2d", "large"])
 def test_host_order(name, which):
-    case = dict(_small_cases())[name]
+    """"large" has more particles than are reordered by one launch a state."""
+    case = dict(_small_cases()).get(name) or cases.fluid_block(2, 560, dx=1e-3, precision=abi.PREC_MIXED, H_fac=2.0)
     print(f"[fields] {name} n={case.n}", flush=True)
     eng = _engine(case)
     x0, dim = eng.field("X"), case.settings.dim

@@ -136,3 +136,24 @@ def test_block_shapes(cells, targets, precision):
     assert same_neighbour_sets(off_e, idx_e, off_o, idx_o)
     assert np.array_equal(eng.neighbour_counts(), np.diff(off_e))
     eng.close()
+
+
+@pytest.mark.parametrize("cells", [2, 2047, 2048, 2049, 4096, 4097, 600_000])
+def test_cell_scan(cells):
+    """Lists of two clusters at the ends of a row of cells: the cell counts'
+    scan at its tiles' edges (2048 cells), one tile to several hundred."""
+    c = _clusters(2, (13,), abi.PREC_FP64, 0)
+    k = len(c.x) // 2
+    cs = 4 * c.settings.particle_step * (1.0 + 1e-7)
+    c.x -= c.x.min(axis=0)
+    c.x[:, 1] *= 1e-3
+    c.x[:, 0] = np.where(np.arange(len(c.x)) < k, c.x[:, 0] % (0.5 * cs), c.x[:, 0] % (0.5 * cs) + (cells - 0.75) * cs)
+    c.x[0, 0], c.x[k, 0] = 0.0, (cells - 0.9) * cs
+    print(f"[walk] scan of {cells} cells n={c.n}", flush=True)
+    eng, orc = _engine(c), _oracle(c)
+    eng.build_neighbours()
+    orc.build_neighbours()
+    off_e, idx_e = eng.neighbours()
+    off_o, idx_o, _ = orc.neighbours()
+    assert same_neighbour_sets(off_e, idx_e, off_o, idx_o)
+    eng.close()
