@@ -42,15 +42,21 @@ template <int D>
 __global__ __launch_bounds__(TPB) void k_bbox_final(const double* partial, int nparts, double* out)
 {
     __shared__ double lds[NWAVE];
+    /* one block: bound by its loads' latency, so all columns of four rows
+     * at once (a column at a time, 16k rows took 56 us) */
+    double v[2 * D];
+#pragma unroll
+    for (int k = 0; k < 2 * D; ++k) v[k] = partial[k];
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nparts; b += TPB)
+#pragma unroll
+        for (int k = 0; k < 2 * D; ++k) {
+            const double w = partial[b * 2 * D + k];
+            v[k] = k < D ? fmin(v[k], w) : fmax(v[k], w);
+        }
 #pragma unroll
     for (int k = 0; k < 2 * D; ++k) {
-        const bool is_min = k < D;
-        double v = partial[k];
-        for (int b = threadIdx.x; b < nparts; b += TPB) {
-            const double w = partial[b * 2 * D + k];
-            v = is_min ? fmin(v, w) : fmax(v, w);
-        }
-        const double r = is_min ? block_reduce(v, OpMin(), lds) : block_reduce(v, OpMax(), lds);
+        const double r = k < D ? block_reduce(v[k], OpMin(), lds) : block_reduce(v[k], OpMax(), lds);
         if (threadIdx.x == 0) out[k] = r;
     }
 }
@@ -486,7 +492,16 @@ __global__ __launch_bounds__(TPB) void k_sum_partials(const double* partial, int
     __shared__ double lds[NWAVE];
     for (int w = 0; w < width; ++w) {
         double v = 0.0;
-        for (int b = threadIdx.x; b < nparts; b += TPB) v += partial[(int64_t)b * width + w];
+        int b = threadIdx.x;
+        /* added up in the rows' order, eight of them asked for at once */
+        for (; b + 7 * TPB < nparts; b += 8 * TPB) {
+            double q[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) q[k] = partial[(int64_t)(b + k * TPB) * width + w];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v += q[k];
+        }
+        for (; b < nparts; b += TPB) v += partial[(int64_t)b * width + w];
         const double r = block_reduce(v, OpSum(), lds);
         if (threadIdx.x == 0) out[w] = r * scale;
     }
@@ -547,13 +562,19 @@ __global__ __launch_bounds__(TPB) void k_dt_reduce(Consts c, DevState s, const i
 __global__ __launch_bounds__(TPB) void k_dt_final(const double* partial, int nparts, double* out)
 {
     __shared__ double lds[NWAVE];
-    for (int k = 0; k < 7; ++k) {
-        double v = partial[k];
-        for (int b = threadIdx.x; b < nparts; b += TPB) {
+    double v[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) v[k] = partial[k];
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nparts; b += TPB) /* as k_bbox_final */
+#pragma unroll
+        for (int k = 0; k < 7; ++k) {
             const double w = partial[b * 7 + k];
-            v = (k < 6) ? fmax(v, w) : fmin(v, w);
+            v[k] = k < 6 ? fmax(v[k], w) : fmin(v[k], w);
         }
-        const double r = (k < 6) ? block_reduce(v, OpMax(), lds) : block_reduce(v, OpMin(), lds);
+#pragma unroll
+    for (int k = 0; k < 7; ++k) {
+        const double r = k < 6 ? block_reduce(v[k], OpMax(), lds) : block_reduce(v[k], OpMin(), lds);
         if (threadIdx.x == 0) out[k] = r;
     }
 }
