@@ -1013,9 +1013,15 @@ __global__ __launch_bounds__(PTPB) void k_dsph_t(Consts c, DevState s, Aux ax, T
  * 20 B of LDS per candidate (36 B with build positions).  A target with
  * fewer than 2 D neighbours takes its pairs in FP64 from the global state
  * (dsph_pair), so the rank test of its correction matrix, which decides
- * between L^-1 and the identity, sees the matrix of the FP64 path. */
+ * between L^-1 and the identity, sees the matrix of the FP64 path.
+ *
+ * Four waves per SIMD: the two pairs' terms fit their 128 registers, while a
+ * fifth wave spilled 112 B a lane into the pair loop (268k particles 0.267 ->
+ * 0.243 ms a launch, 700k 0.563 -> 0.499, 4M 2.60 -> 2.32).  The surface
+ * loops do better with five, spilling as they do (268k 0.582 ms together,
+ * 0.610 with four). */
 #ifndef FJ_DSPH_OCC
-#define FJ_DSPH_OCC __attribute__((amdgpu_waves_per_eu(5, 8)))
+#define FJ_DSPH_OCC __attribute__((amdgpu_waves_per_eu(4, 8)))
 #endif
 template <int D, bool FR>
 __global__ __launch_bounds__(PTPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s, Aux ax, TileGrid tg, NbrList nl, double* partial)
