@@ -731,10 +731,11 @@ void group_blocks(fjsph_ctx* ctx)
  * fastest for large sets; below a few hundred thousand particles it leaves
  * too few blocks for 256 CUs, and blocks of 128 and 64, whose waves share
  * the lists (Split), win although they stage more.  ms a step with 256 / 128
- * / 64 targets, 3D: 100k Runge-Kutta 4.14 / 3.18 / 3.09, 268k 12.9 / 11.5 /
- * 11.4, 700k 9.00 / 8.98 / 10.9, 1M 14.4 / 14.7 / 18.2.  In 2D a target has a tenth of the neighbours, so blocks are
- * shorter work and the line lies lower: 6.5k 1.24 / 1.13 / 1.16, 86k 1.39 /
- * 1.41 / 1.56, 345k 2.04 / 2.39 / 2.99.  FP64 keeps its blocks, see
+ * / 64 targets, 3D: 100k Runge-Kutta 3.15 / 2.33 / 2.24, 268k 11.3 / 9.9 /
+ * 9.7, 700k 7.83 / 7.76 / 9.00, 1M 12.6 / 12.7 / 15.2.  In 2D a target has
+ * a tenth of the neighbours, so blocks are shorter work and the line lies
+ * lower: 23k 0.98 / 0.96 / 0.91, 92k 1.14 / 1.17 / 1.26, 345k 1.80 / 2.08 /
+ * 2.59.  FP64 keeps its blocks, see
  * block_shape. */
 int32_t default_targets(int dim, int64_t n, bool f32)
 {

@@ -1016,8 +1016,8 @@ __global__ __launch_bounds__(PTPB) void k_dsph_t(Consts c, DevState s, Aux ax, T
  * between L^-1 and the identity, sees the matrix of the FP64 path.
  *
  * Four waves per SIMD: the two pairs' terms fit their 128 registers, while a
- * fifth wave spilled 112 B a lane into the pair loop (268k particles 0.267 ->
- * 0.243 ms a launch, 700k 0.563 -> 0.499, 4M 2.60 -> 2.32).  The surface
+ * fifth wave spilled 112 B a lane into the pair loop (the whole pass: 268k
+ * particles 0.267 -> 0.243 ms, 700k 0.563 -> 0.499, 4M 2.60 -> 2.32).  The surface
  * loops do better with five, spilling as they do (268k 0.582 ms together,
  * 0.610 with four). */
 #ifndef FJ_DSPH_OCC
@@ -3211,9 +3211,9 @@ __device__ void skin_friction(const Consts& c, const double* Vd, const double* n
 
 
 /* Occupancy request for the force passes: four waves per SIMD.  With two
- * records in flight the pass is bound by vector issue (0.94 instructions per
- * CU-cycle at 4M particles), and a fifth wave only spills: 2.57 ms a launch
- * against 2.74. */
+ * records in flight the pass is bound by vector issue (0.85 instructions per
+ * CU-cycle at 1M particles, 12% of the CU time the launch's end), and a fifth
+ * wave only spills: 2.57 ms a launch at 4M against 2.74 (2.46 now). */
 #ifndef FJ_FORCE_OCC
 #define FJ_FORCE_OCC __attribute__((amdgpu_waves_per_eu(4, 8)))
 #endif
