@@ -403,11 +403,17 @@ struct Rows {
 /* FJ_TILE_PAIRS_BEGIN(cu, nl, base, P) { body } FJ_TILE_PAIRS_END(cu, nl):
  * the same walk, P (1, 2 or 4) entries of a row at a time and without a
  * branch per entry: `t[e]` is the tile-local index of entry e and `ok[e]`
- * whether there is one (t[e] = 0, a staged slot, otherwise), so the body can
- * read the P records before it uses the first of them and masks the terms of
- * a missing entry itself: its weight is zero, and where a factor of a pair
- * could overflow at a slot far outside the support (the fourth power of W in
- * the shift) its distance too.  Entries fill a row from its low end. */
+ * whether there is one, so the body can read the P records before it uses
+ * the first of them.  A missing entry reads NONE, a record of zeros behind
+ * the tile's (the kernel writes it once): its weight is zero and every other
+ * value finite, so that it adds nothing whatever the particles of the tile
+ * hold (a staged slot's values times zero would spread a NaN to targets that
+ * are no neighbours of it).  The body masks what a record of zeros does not:
+ * W itself, maxima, and the distance where a factor of a pair could overflow
+ * at a slot far outside the support (the fourth power of W in the shift).
+ * Entries fill a row from its low end. */
+constexpr int NONE = TILE;
+static_assert(NO_ENTRY >= (NO_ENTRY / TILE - 1) * TILE + TILE, "NO_ENTRY lies past every tile's slots");
 #define FJ_TILE_PAIRS_BEGIN(cu, nl, base, P)                                              \
     for (;;) {                                                                            \
         const bool fj_act = (cu).row_in(uint32_t((base) + TILE));                         \
@@ -422,7 +428,7 @@ struct Rows {
             {                                                                             \
                 const uint32_t fj_uq = uint32_t(fj_u >> (16 * e)) & 0xFFFFu;              \
                 ok[e] = fj_uq != NO_ENTRY;                                                \
-                t[e] = ok[e] ? int(fj_uq) - (base) : 0;                                   \
+                t[e] = int(min(fj_uq - uint32_t(base), uint32_t(NONE)));                  \
             }                                                                             \
             if (!__any(ok[0])) break;                                                     \
             fj_u = (P) < 4 ? fj_u >> (16 * ((P) & 3)) : ~0ull;
@@ -945,11 +951,18 @@ template <int D, bool FR>
 __global__ __launch_bounds__(PTPB) void k_dsph_t(Consts c, DevState s, Aux ax, TileGrid tg, NbrList nl, double* partial)
 {
     constexpr int NS = D * (D + 1) / 2;
-    __shared__ double tp[D][TILE];
-    __shared__ double tvol[TILE], trho[TILE];
-    __shared__ int32_t tnb[TILE], tsl[FR ? TILE : 1];
+    __shared__ double tp[D][TILE + 1];
+    __shared__ double tvol[TILE + 1], trho[TILE + 1];
+    __shared__ int32_t tnb[TILE + 1], tsl[FR ? TILE + 1 : 1];
     __shared__ BlockHead h;
     __shared__ double lds[PWAVE];
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) tp[a][NONE] = 0.0;
+        tvol[NONE] = trho[NONE] = 0.0;
+        tnb[NONE] = 0;
+        if constexpr (FR) tsl[NONE] = 0;
+    }
     block_head<D>(tg, h);
     const int U = h.U;
     const int NT = n_tiles(U);
@@ -996,8 +1009,9 @@ __global__ __launch_bounds__(PTPB) void k_dsph_t(Consts c, DevState s, Aux ax, T
 #pragma unroll
                 for (int a = 0; a < D; ++a) xj[a] = tp[a][t[0]];
                 frozen_r<D, FR>(xi, xj, xbi, ax.xb, FR ? tsl[FR ? t[0] : 0] : 0, d2, r);
-                npd_acc += dsph_pair<D>(c, inv_H, xi, xj, r, ok[0] ? tvol[t[0]] : 0.0, trho[t[0]],
-                                        ok[0] && tnb[t[0]] != 0, rhoi, Lm, Lnb, gR, nr, kernsum, colour);
+                if (FR && !ok[0]) r = 0.0; /* NONE has no build position of its own */
+                npd_acc += dsph_pair<D>(c, inv_H, xi, xj, r, tvol[t[0]], trho[t[0]], tnb[t[0]] != 0, rhoi, Lm, Lnb, gR,
+                                        nr, kernsum, colour);
             FJ_TILE_PAIRS_END(cu, nl)
         }
         dsph_fold<D>(sp, &tp[0][0], Lm, Lnb, gR, nr, kernsum, colour);
@@ -1027,12 +1041,17 @@ template <int D, bool FR>
 __global__ __launch_bounds__(PTPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState s, Aux ax, TileGrid tg, NbrList nl, double* partial)
 {
     constexpr int NS = D * (D + 1) / 2;
-    __shared__ float4 tA[TILE];            /* x_j - xref, +V_j (-V_j: j is PISTON or BOUND) */
-    __shared__ float tR[TILE];             /* rho_j - rref */
-    __shared__ float4 tX[FR ? TILE : 1];   /* xb_j - xbref */
+    __shared__ float4 tA[TILE + 1];          /* x_j - xref, +V_j (-V_j: j is PISTON or BOUND) */
+    __shared__ float tR[TILE + 1];           /* rho_j - rref */
+    __shared__ float4 tX[FR ? TILE + 1 : 1]; /* xb_j - xbref */
     __shared__ BlockHead h;
-    __shared__ int32_t has_wall;           /* a PISTON or BOUND slot was staged */
-    if (threadIdx.x == 0) has_wall = 0;
+    __shared__ int32_t has_wall;             /* a PISTON or BOUND slot was staged */
+    if (threadIdx.x == 0) {
+        has_wall = 0;
+        tA[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+        tR[NONE] = 0.f;
+        if constexpr (FR) tX[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
     __shared__ double lds[PWAVE];
     block_head<D>(tg, h);
     const int U = h.U;
@@ -1141,7 +1160,7 @@ __global__ __launch_bounds__(PTPB) FJ_DSPH_OCC void k_dsph_m(Consts c, DevState 
                          * with r from the current positions R is zero there */
                         const float t3 = (FR && r < 1e-12f) ? 0.f : t2 * tq;
                         const float w = ok[e] ? t2 * t2 * fmaf(r, 2.f, 1.f) : 0.f;
-                        const float sv = ok[e] ? A.w : 0.f;
+                        const float sv = A.w;
                         const float volj = WALL ? fabsf(sv) : sv;
                         const float cc = volj * t3;
                         const float drho = (Re[e] - drhoi) - rlo;
@@ -1630,14 +1649,23 @@ __global__ __launch_bounds__(PTPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevS
 {
     constexpr bool with_surf = MODE != 2;
     constexpr bool with_diss = MODE != 0;
-    constexpr int TD = with_diss ? TILE : 1;
-    __shared__ float4 tA[TILE];            /* x_j - xref, V_j            */
-    __shared__ float4 tB[TILE];            /* v_j - vref, lambda_j       */
-    __shared__ float4 tG[TD];              /* gradRho_j, rho_j - rref    */
-    __shared__ float2 tE[TD];              /* sqrt(B gam / rho_j), m_j (negative: j is PISTON or BOUND) */
-    __shared__ float4 tX[FR ? TILE : 1];   /* xb_j - xbref               */
+    constexpr int TD = with_diss ? TILE + 1 : 1;
+    __shared__ float4 tA[TILE + 1];          /* x_j - xref, V_j            */
+    __shared__ float4 tB[TILE + 1];          /* v_j - vref, lambda_j       */
+    __shared__ float4 tG[TD];                /* gradRho_j, rho_j - rref    */
+    __shared__ float2 tE[TD];                /* sqrt(B gam / rho_j), m_j (negative: j is PISTON or BOUND) */
+    __shared__ float4 tX[FR ? TILE + 1 : 1]; /* xb_j - xbref               */
     __shared__ int32_t tsl[with_surf ? TILE : 1];
     __shared__ BlockHead h;
+    if (threadIdx.x == 0) {
+        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+        tA[NONE] = tB[NONE] = zero;
+        if constexpr (with_diss) {
+            tG[NONE] = zero;
+            tE[NONE] = make_float2(0.f, 0.f);
+        }
+        if constexpr (FR) tX[NONE] = zero;
+    }
     block_head<D>(tg, h);
     const int U = h.U;
     const int NT = n_tiles(U);
@@ -1786,7 +1814,7 @@ __global__ __launch_bounds__(PTPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevS
                 const float tq = fmaf(r, ktq, 1.f);
                 const float t3 = (FR && r < rmin) ? 0.f : tq * tq * tq;
                 const float4 B = Be[e];
-                const float vt = (ok[e] ? A.w : 0.f) * t3;
+                const float vt = A.w * t3;
                 if constexpr (with_surf) {
                     if (testing && !found && ok[e]) {
                         /* point-T test (src/Geometry.cpp:43-98) in FP32 unless
@@ -1851,7 +1879,7 @@ __global__ __launch_bounds__(PTPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevS
                         vdotr += ((vj[a] - vit[a]) - vlo[a]) * Rji[a];
                         gsum += (gri[a] + grj[a]) * Rji[a];
                     }
-                    const float mj = ok[e] ? fmaxf(E.y, 0.f) : 0.f;
+                    const float mj = fmaxf(E.y, 0.f);
                     const float ff = (mj * (cfac + E.x)) * (fminf(vdotr, 0.f) * idist2) *
                                      (fast_rcp<float>(fmaf(0.5f, G.w, rhom)) * t3);
 #pragma unroll
@@ -2110,10 +2138,14 @@ template <int D, bool FR>
 __global__ __launch_bounds__(PTPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
                                                     TileGrid tg, NbrList nl, const double* __restrict__ norms_tmp)
 {
-    __shared__ float4 tA[TILE];            /* x_j - xref, V_j */
-    __shared__ float4 tN[TILE];            /* surface normal of j (Detect_Surface loop 1), surf_j */
-    __shared__ float4 tX[FR ? TILE : 1];   /* xb_j - xbref */
+    __shared__ float4 tA[TILE + 1];          /* x_j - xref, V_j */
+    __shared__ float4 tN[TILE + 1];          /* surface normal of j (Detect_Surface loop 1), surf_j */
+    __shared__ float4 tX[FR ? TILE + 1 : 1]; /* xb_j - xbref */
     __shared__ BlockHead h;
+    if (threadIdx.x == 0) {
+        tA[NONE] = tN[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (FR) tX[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
     block_head<D>(tg, h);
     const int U = h.U;
     const int NT = n_tiles(U);
@@ -2219,7 +2251,7 @@ __global__ __launch_bounds__(PTPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevS
                 bool nj_nz = false;
 #pragma unroll
                 for (int a = 0; a < D; ++a) nj_nz = nj_nz || nj[a] != 0.f;
-                if (ok[e] && ni_nz && nj_nz) {
+                if (ni_nz && nj_nz) {
                     float W, fg;
                     wendland<float>(r, Ht, inv_Hf, Wcf, W, fg);
                     float tt = 0.f;
@@ -2239,7 +2271,7 @@ __global__ __launch_bounds__(PTPB) FJ_SURF2_OCC void k_surface2_m(Consts c, DevS
                     q = -q / r;
                     if (q > qmax) qmax = q;
                 }
-                zone = zone || (ok[e] && N.w != 0.f);
+                zone = zone || N.w != 0.f;
                 }
             FJ_TILE_PAIRS_END(cu, nl)
             curve += double(fcurve);
@@ -2440,11 +2472,15 @@ template <int D, bool FR>
 __global__ __launch_bounds__(PTPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevState s, Aux ax, const int32_t* __restrict__ part_id,
                                                  TileGrid tg, NbrList nl)
 {
-    __shared__ float4 tA[TILE];            /* x_j - xref, +V_j (-V_j: j is PISTON or BOUND) */
-    __shared__ float4 tV[TILE];            /* v_j - vref */
-    __shared__ double tn[D][TILE];         /* normalised normal of j */
-    __shared__ float4 tX[FR ? TILE : 1];   /* xb_j - xbref */
+    __shared__ float4 tA[TILE + 1];          /* x_j - xref, +V_j (-V_j: j is PISTON or BOUND) */
+    __shared__ float4 tV[TILE + 1];          /* v_j - vref */
+    __shared__ double tn[D][TILE];           /* normalised normal of j */
+    __shared__ float4 tX[FR ? TILE + 1 : 1]; /* xb_j - xbref */
     __shared__ BlockHead h;
+    if (threadIdx.x == 0) {
+        tA[NONE] = tV[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (FR) tX[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
     block_head<D>(tg, h);
     const int U = h.U;
     const int NT = n_tiles(U);
@@ -2539,7 +2575,7 @@ __global__ __launch_bounds__(PTPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevStat
                 wendland<float>(fast_sqrt<float>(rr), Ht, inv_Hf, Wcf, W, fg);
                 const float w = W * inv_Wdx;
                 const float w2 = w * w;
-                const float f = (1.f + 0.2f * (w2 * w2)) * fg * (ok[e] ? fabsf(A.w) : 0.f);
+                const float f = (1.f + 0.2f * (w2 * w2)) * fg * fabsf(A.w);
                 float dv2 = 0.f;
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
@@ -2547,7 +2583,7 @@ __global__ __launch_bounds__(PTPB) FJ_SHIFT_OCC void k_shift_m(Consts c, DevStat
                     const float dv = (vj[a] - vit[a]) - vlo[a];
                     dv2 += dv * dv;
                 }
-                if (ok[e] && A.w > 0.f) {
+                if (A.w > 0.f) {
                     double d = 0.0;
 #pragma unroll
                     for (int a = 0; a < D; ++a) d += nhat[a] * tn[a][t[e]];
@@ -2618,12 +2654,16 @@ __global__ __launch_bounds__(PTPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts
                                                                    const int32_t* __restrict__ part_id, TileGrid tg,
                                                                    NbrList nl, const double* __restrict__ norms_tmp)
 {
-    __shared__ float4 tA[TILE];            /* x_j - xref, +V_j (-V_j: j is PISTON or BOUND) */
-    __shared__ float4 tN[TILE];            /* surface normal of j (Detect_Surface loop 1), surf_j */
-    __shared__ float4 tV[TILE];            /* v_j - vref */
-    __shared__ int32_t tsl[TILE];          /* particle slot of j (FP64 normal of an undecided angle test) */
-    __shared__ float4 tX[FR ? TILE : 1];   /* xb_j - xbref */
+    __shared__ float4 tA[TILE + 1];          /* x_j - xref, +V_j (-V_j: j is PISTON or BOUND) */
+    __shared__ float4 tN[TILE + 1];          /* surface normal of j (Detect_Surface loop 1), surf_j */
+    __shared__ float4 tV[TILE + 1];          /* v_j - vref */
+    __shared__ int32_t tsl[TILE];            /* particle slot of j (FP64 normal of an undecided angle test) */
+    __shared__ float4 tX[FR ? TILE + 1 : 1]; /* xb_j - xbref */
     __shared__ BlockHead h;
+    if (threadIdx.x == 0) {
+        tA[NONE] = tN[NONE] = tV[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (FR) tX[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
     block_head<D>(tg, h);
     const int U = h.U;
     const int NT = n_tiles(U);
@@ -2731,7 +2771,7 @@ __global__ __launch_bounds__(PTPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts
                 for (int e = 0; e < kPairs; ++e) {
                 const float4 A = Ae[e], N = Ne[e];
                 const float pj[3] = {A.x, A.y, A.z}, nj[3] = {N.x, N.y, N.z};
-                const float sv = ok[e] ? A.w : 0.f;
+                const float sv = A.w;
                 const float volj = fabsf(sv);
                 float Rij[D], rr;
 #pragma unroll
@@ -2781,7 +2821,7 @@ __global__ __launch_bounds__(PTPB) FJ_SURF2SHIFT_OCC void k_surf2_shift_m(Consts
                     q = -q * fast_rcp<float>(r);
                     if (q > qmax) qmax = q;
                 }
-                zone = zone || (ok[e] && N.w != 0.f);
+                zone = zone || N.w != 0.f;
                 /* particle_shift */
                 if (work) {
                     const float4 V = Ve[e];
@@ -3402,7 +3442,7 @@ __global__ __launch_bounds__(PTPB) void k_force_t(Consts c, DevState s, Aux ax,
  *   V_j = |m_j| / rho_j is formed as |m_j| * (1/rho_j). */
 template <bool ALE>
 struct ForceTileM {
-    float4 A[TILE], B[TILE], X[TILE], E[ALE ? TILE : 1];
+    float4 A[TILE + 1], B[TILE + 1], X[TILE + 1], E[ALE ? TILE + 1 : 1];
 };
 
 /* Mixed-precision form of k_force_t: pair terms in FP32 on coordinates and
@@ -3425,6 +3465,10 @@ __global__ __launch_bounds__(PTPB) FJ_FORCE_OCC void k_force_m(Consts c, DevStat
     constexpr int P = ALE ? kPairs : 1; /* entries taken together (kPairs) */
     __shared__ ForceTileM<ALE> ft;
     __shared__ BlockHead h;
+    if (threadIdx.x == 0) {
+        ft.A[NONE] = ft.B[NONE] = ft.X[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (ALE) ft.E[NONE] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
     block_head<D>(tg, h);
     const int U = h.U;
     const int NT = n_tiles(U);
@@ -3544,7 +3588,7 @@ __global__ __launch_bounds__(PTPB) FJ_FORCE_OCC void k_force_m(Consts c, DevStat
                     for (int a = 1; a < D; ++a) rr += Rji[a] * Rji[a];
                 }
                 const float r = fast_sqrt<float>(rr);
-                const float msg = ok[e] ? A.w : 0.f, Pj = B.w, irj = X.w;
+                const float msg = A.w, Pj = B.w, irj = X.w;
                 const bool bound_j = msg < 0.f;
                 const float mj = fabsf(msg);
                 const float volj = mj * irj;

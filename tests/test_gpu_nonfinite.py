@@ -1,0 +1,85 @@
+"""Non-finite values stay where the pair sums put them: a NaN of one particle
+reaches that particle and its neighbours in the pass that reads it, whatever
+rows and tiles the other particles share with it."""
+import numpy as np
+import pytest
+
+from fjsph_amd import abi, cases
+from tests.test_gpu_parity import _engine
+
+pytestmark = pytest.mark.gpu
+
+
+def _cloud(dim, precision, ale=0):
+    """A fluid block of several cells along each axis, with lists of many
+    lengths (inner particles and faces)."""
+    c = cases.fluid_block(dim, 40 if dim == 2 else 12, dx=1e-3, precision=precision, jitter=0.1, seed=3, H_fac=1.5,
+                          sig=0.07)
+    s = c.settings
+    s.ale, s.mu, s.visc_alpha = ale, 1e-3, 0.1
+    rng = np.random.default_rng(23)
+    c.v = rng.uniform(-0.1, 0.1, c.x.shape)
+    c.rho = s.rho_rest * (1.0 + rng.uniform(-5e-3, 5e-3, c.n))
+    b = s.rho_rest * s.speed_sound ** 2 / s.gam
+    c.p = b * ((c.rho / s.rho_rest) ** s.gam - 1.0)
+    return c
+
+
+def _reached(off, idx, k):
+    """Particle k and those it is a neighbour of (the sets are symmetric)."""
+    r = np.zeros(len(off) - 1, bool)
+    r[k] = True
+    r[idx[off[k]:off[k + 1]]] = True
+    return r
+
+
+def _first_of_cells(c):
+    """The lowest particle of every cell (edge 2 H): a tile block's mixed
+    sums are relative to its first target, which is one of them."""
+    cs = 2.0 * c.settings.H_fac * c.settings.particle_step * (1.0 + 1e-7)
+    cell = np.floor((c.x - c.x.min(axis=0)) / cs).astype(np.int64)
+    return set(np.unique(cell, axis=0, return_index=True)[1].tolist())
+
+
+def _nonfinite(a):
+    return ~np.isfinite(a.reshape(len(a), -1)).all(axis=1)
+
+
+@pytest.mark.parametrize("precision", [abi.PREC_FP64, abi.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("targets", [16, 256])
+@pytest.mark.parametrize("dim,ale", [(2, 0), (3, 0), (3, 1)], ids=["2d", "3d", "3d-ale"])
+def test_nan_reaches_neighbours_only(dim, ale, targets, precision):
+    """Rows of four entries are filled up with entries that are none: they
+    must not carry the values of a particle that is no neighbour.  (A NaN in
+    the reference of a block's FP32 coordinates reaches the whole block.)"""
+    c = _cloud(dim, precision, ale)
+    print(f"[nonfinite] {dim}D ale={ale} n={c.n} {targets} targets a block precision={precision}", flush=True)
+    eng = _engine(c)
+    eng.set_block_targets(targets)
+    eng.build_neighbours()
+    off, idx = eng.neighbours()
+    npd = eng.dsph_prestep()
+    rho, v = eng.field("RHO"), eng.field("V")
+    skip = _first_of_cells(c) if precision == abi.PREC_MIXED else ()
+    for k in range(0, c.n, 5 if dim == 2 else 7):
+        if k in skip:
+            continue
+        near = _reached(off, idx, k)
+        bad = rho.copy()
+        bad[k] = np.nan
+        eng.set_field("RHO", bad)
+        eng.dsph_prestep()
+        for f in ("KERNSUM", "COLOUR", "GRADRHO"):
+            assert not (_nonfinite(eng.field(f)) & ~near).any(), (f, k)
+        eng.set_field("RHO", rho)
+        eng.dsph_prestep()
+        bad = v.copy()
+        bad[k] = np.nan
+        eng.set_field("V", bad)
+        eng.dissipation_terms()
+        eng.acc_rrho(npd)
+        for f in ("AVISC", "ACC", "RRHO"):
+            assert not (_nonfinite(eng.field(f)) & ~near).any(), (f, k)
+        eng.set_field("V", v)
+        eng.dissipation_terms()
+    eng.close()
