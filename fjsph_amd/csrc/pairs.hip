@@ -1869,8 +1869,9 @@ __global__ __launch_bounds__(PTPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevS
                     const float idist2 = fast_rcp<float>(rr + eps2);
                     const float drho = (G.w - drhoi) - rlo;
                     /* artificial viscosity of an approaching pair, none with a
-                     * wall particle (E.y is negative then); without a branch,
-                     * which nearly every wave took: the surface loops together
+                     * wall particle (E.y is negative then), a NaN velocity
+                     * of a fluid pair handed on; without a branch, which
+                     * nearly every wave took: the surface loops together
                      * 0.640 -> 0.586 ms (268k particles), 1.50 -> 1.38 (1M) */
                     float vdotr = ((vj[0] - vit[0]) - vlo[0]) * Rji[0];
                     float gsum = (gri[0] + grj[0]) * Rji[0];
@@ -1879,9 +1880,9 @@ __global__ __launch_bounds__(PTPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevS
                         vdotr += ((vj[a] - vit[a]) - vlo[a]) * Rji[a];
                         gsum += (gri[a] + grj[a]) * Rji[a];
                     }
-                    const float mj = fmaxf(E.y, 0.f);
-                    const float ff = (mj * (cfac + E.x)) * (fminf(vdotr, 0.f) * idist2) *
-                                     (fast_rcp<float>(fmaf(0.5f, G.w, rhom)) * t3);
+                    const bool wet = E.y > 0.f;
+                    float ff = (E.y * (cfac + E.x)) * (vdotr * idist2) * (fast_rcp<float>(fmaf(0.5f, G.w, rhom)) * t3);
+                    ff = wet && !(vdotr > 0.f) ? ff : 0.f;
 #pragma unroll
                     for (int a = 0; a < D; ++a) fav[a] = fmaf(ff, Rji[a], fav[a]);
                     /* R . grad W = W'(r)/r R . R */
@@ -1891,7 +1892,7 @@ __global__ __launch_bounds__(PTPB) FJ_SURF1_OCC void k_surface1_m(Consts c, DevS
 #pragma unroll
                         for (int a = 1; a < D; ++a) R2 += Rji[a] * Rji[a];
                     }
-                    frd = fmaf((vt * R2) * idist2, fmaf(E.y > 0.f ? 0.5f : 0.f, gsum, drho), frd);
+                    frd = fmaf((vt * R2) * idist2, fmaf(0.5f, wet ? gsum : 0.f, drho), frd);
                 }
                 }
             FJ_TILE_PAIRS_END(cu, nl)

@@ -83,3 +83,30 @@ def test_nan_reaches_neighbours_only(dim, ale, targets, precision):
         eng.set_field("V", v)
         eng.dissipation_terms()
     eng.close()
+
+
+@pytest.mark.parametrize("precision", [abi.PREC_FP64, abi.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_nan_velocity_enters_the_viscosity(dim, precision):
+    """An approach speed that is NaN gives a NaN viscosity of every fluid
+    particle in reach, no viscosity next to a wall."""
+    c = _cloud(dim, precision)
+    wall = 5
+    c.b[wall], c.n_bound = abi.BOUND, wall + 1
+    c.blocks = [dict(first=0, last=wall + 1, is_fluid=0, bound_solver=abi.DBC),
+                dict(first=wall + 1, last=c.n, is_fluid=1)]
+    print(f"[nonfinite] viscosity {dim}D n={c.n} precision={precision}", flush=True)
+    eng = _engine(c)
+    eng.build_neighbours()
+    off, idx = eng.neighbours()
+    eng.dsph_prestep()
+    v = eng.field("V")
+    for k in (wall, *[k for k in range(wall + 1, c.n, c.n // 5) if k not in _first_of_cells(c)]):
+        bad = v.copy()
+        bad[k] = np.nan
+        eng.set_field("V", bad)
+        eng.dissipation_terms()
+        want = _reached(off, idx, k) if k != wall else np.zeros(c.n, bool)
+        got = _nonfinite(eng.field("AVISC"))
+        assert np.array_equal(got[wall + 1:], want[wall + 1:]), k
+    eng.close()
