@@ -497,6 +497,7 @@ __device__ __forceinline__ float wave_maxf(float v)
  * by word: the whole neighbour pass of 268k particles 0.505 -> 0.392 ms, of
  * 700k 0.793 -> 0.688, of 200k in FP64 0.446 -> 0.351. */
 constexpr int WORDS = (TILE + 31) / 32;
+constexpr float kFar = 1e30f; /* |y|^2 of a slot that is nobody's neighbour */
 
 template <int D>
 __global__ __launch_bounds__(PTPB) void k_build_t(const double* __restrict__ x, TileGrid tg, double sr, double inv_r,
@@ -560,6 +561,11 @@ __global__ __launch_bounds__(PTPB) void k_build_t(const double* __restrict__ x, 
             blo[a] = wave_minf(active ? xit[a] : HUGE_VALF);
             bhi[a] = wave_maxf(active ? xit[a] : -HUGE_VALF);
         }
+        if (!(cx < kFar)) { /* a NaN position, whose sign would decide: no neighbours */
+            cx = kFar;
+#pragma unroll
+            for (int a = 0; a < D; ++a) m2x[a] = 0.f;
+        }
         /* the target's own slot in the union (tile k_self, slot t_self):
          * the segment of the block's own cell row holds its order position */
         int k_self = -1, t_self = 0;
@@ -582,7 +588,7 @@ __global__ __launch_bounds__(PTPB) void k_build_t(const double* __restrict__ x, 
                 const int u = tile_union_index(tk, t, NT);
                 if (u >= U) {
                     /* padding: never a neighbour */
-                    tf[t] = make_float4(0.f, 0.f, 0.f, 1e30f);
+                    tf[t] = make_float4(0.f, 0.f, 0.f, kFar);
                     continue;
                 }
                 const int32_t sl = union_slot(tg, h.ut, u);
@@ -593,7 +599,8 @@ __global__ __launch_bounds__(PTPB) void k_build_t(const double* __restrict__ x, 
                     pa[a] = float((tp[a][t] - xref[a]) * inv_r);
                     y2 = fmaf(pa[a], pa[a], y2);
                 }
-                tf[t] = make_float4(pa[0], pa[1], pa[2], y2);
+                /* a NaN position: nobody's neighbour */
+                tf[t] = y2 < kFar ? make_float4(pa[0], pa[1], pa[2], y2) : make_float4(0.f, 0.f, 0.f, kFar);
             }
             __syncthreads();
             /* groups of 4 slots with a candidate in reach of the wave's
@@ -615,7 +622,7 @@ __global__ __launch_bounds__(PTPB) void k_build_t(const double* __restrict__ x, 
                             const float da = fmaxf(fmaxf(blo[a] - pp[a], pp[a] - bhi[a]), 0.f);
                             d2b += da * da;
                         }
-                        reach = reach || (d2b <= 1.f + band && P.w < 1e30f);
+                        reach = reach || (d2b <= 1.f + band && P.w < kFar);
                     }
                 }
                 gmask[hgrp] = __ballot(reach);

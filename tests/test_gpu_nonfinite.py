@@ -110,3 +110,26 @@ def test_nan_velocity_enters_the_viscosity(dim, precision):
         got = _nonfinite(eng.field("AVISC"))
         assert np.array_equal(got[wall + 1:], want[wall + 1:]), k
     eng.close()
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0], ids=["+nan", "-nan"])
+@pytest.mark.parametrize("precision", [abi.PREC_FP64, abi.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_nan_position_is_nobodys_neighbour(dim, precision, sign):
+    """Whatever its sign (x86 makes NaNs with the sign set)."""
+    c = _cloud(dim, precision)
+    print(f"[nonfinite] position {dim}D n={c.n} precision={precision} sign={sign}", flush=True)
+    eng = _engine(c)
+    eng.build_neighbours()
+    off, idx = eng.neighbours()
+    k = c.n - 1
+    keep = np.array([[j for j in idx[off[i]:off[i + 1]] if j != k] for i in range(k)], dtype=object)
+    eng.close()
+    c.x[k] = np.copysign(np.nan, sign)
+    eng = _engine(c)
+    eng.build_neighbours()
+    off, idx = eng.neighbours()
+    for i in range(k):
+        assert list(idx[off[i]:off[i + 1]]) == list(keep[i]), i
+    assert list(idx[off[k]:]) == [k]
+    eng.close()
