@@ -55,7 +55,7 @@ METRIC = "particle-steps/s and %HBM roofline at 4M 3D particles; surrogate vs me
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_force_m_jet4m_traffic.json")
 
 
-AUTOTUNE_CANDIDATES = (128, 192, 256, 384, 512, 768, 1024)
+AUTOTUNE_CANDIDATES = (64, 128, 192, 256, 384, 512, 768, 1024)
 
 
 def workload(name, n_target):
@@ -201,8 +201,9 @@ def run_engine(case, args, label, autotune=True, block_targets=None, steps=None)
         # control, Newmark-Beta convergence and npd
         eng.set_groups(case.owner)
     eng.set_reorder_interval(args.reorder_every)
-    if block_targets or args.block_targets:
-        eng.set_block_targets(block_targets or args.block_targets)
+    set_targets = block_targets or args.block_targets or None
+    if set_targets:
+        eng.set_block_targets(set_targets)
     if getattr(case, "surrogate", None) is not None:
         eng.set_surrogate(case.surrogate)
     eng.integrate_no_update()
@@ -212,6 +213,7 @@ def run_engine(case, args, label, autotune=True, block_targets=None, steps=None)
     if autotune and not args.no_autotune:
         # tile blocks chosen by the engine's autotuner on this state (untimed)
         best, ms = eng.autotune_blocks(AUTOTUNE_CANDIDATES, reps=2)
+        set_targets = best
         tune = {"block_targets": best, "ms_per_candidate": {str(k): v for k, v in ms.items()}}
         print(f"[bench] {label}: autotuned tile blocks: {best} targets per block", file=sys.stderr, flush=True)
         eng.integrate_step()
@@ -232,7 +234,8 @@ def run_engine(case, args, label, autotune=True, block_targets=None, steps=None)
     r = {"elapsed": elapsed, "value": particle_steps / elapsed, "its": float(np.mean(its)), "autotune": tune,
          "window_ns": [w0, w1],
          "particles_end": eng.n,
-         "steps": steps, "block_targets": eng.get_block_targets(),
+         # what ran, and what another run takes to run the same blocks (None: the engine's own choice)
+         "steps": steps, "block_targets": eng.get_block_targets(), "set_targets": set_targets,
          "timers": eng.timers(), "stats": eng.neighbour_stats(),
          "force_bpp": eng.pass_bytes(abi.TIMER_NAMES.index("force")),
          "pass_bytes": {k: eng.pass_bytes(abi.TIMER_NAMES.index(k)) for k in abi.TIMER_NAMES}}
@@ -279,9 +282,9 @@ def main():
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-extra", action="store_true",
                     help="skip the constant-gas and FP64 runs and the error check (profiling runs)")
-    ap.add_argument("--no-autotune", action="store_true", help="keep the tile blocks as set (default 256 targets)")
+    ap.add_argument("--no-autotune", action="store_true", help="keep the tile blocks as set (default: the engine's choice)")
     ap.add_argument("--block-targets", type=int, default=0,
-                    help="targets per tile block before any autotuning (0: the engine's default, 256)")
+                    help="targets per tile block before any autotuning (0: the engine's choice)")
     ap.add_argument("--reorder-every", type=int, default=4,
                     help="steps between the cell-order permutations of the particle arrays")
     ap.add_argument("--copy-probe", type=int, default=0)
@@ -378,7 +381,7 @@ def main():
             # the same state with the constant gas velocity the CPU sample uses
             t0 = time.perf_counter()
             const_run = run_engine(const_case, args, "constant-velocity aero (CPU-comparable)", autotune=False,
-                                   block_targets=run["block_targets"])
+                                   block_targets=run["set_targets"])
             phases["engine_const_s"] = time.perf_counter() - t0
 
     timers = run["timers"]
@@ -438,7 +441,7 @@ def main():
     fp64 = None
     if not args.no_extra:
         t0 = time.perf_counter()
-        fp64 = fp64_check(const_case or case, args, run["block_targets"])
+        fp64 = fp64_check(const_case or case, args, run["set_targets"])
         phases["fp64_and_error_s"] = time.perf_counter() - t0
 
     cpu = None
@@ -526,7 +529,8 @@ def fp64_check(case, args, block_targets):
         eng = Engine(c)
         if grouped:
             eng.set_groups(c.owner)
-        eng.set_block_targets(block_targets)
+        if block_targets:
+            eng.set_block_targets(block_targets)
         # positions the step starts from (the start-up pass leaves a predicted
         # state in place, which the step recomputes from these)
         x_before = dict(zip(eng.field("PID").tolist(), eng.field("X")))

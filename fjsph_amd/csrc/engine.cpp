@@ -125,7 +125,7 @@ struct fjsph_ctx {
     int64_t mesh_ncells = 0;
     std::vector<double> mcentre, mvel, mp, mrho;
     double mesh_max_len = 0.0; /* MESH::maxlength */
-    int32_t block_targets = 0; /* targets per tile block (0: 256) */
+    int32_t block_targets = 0; /* targets per tile block (0: default_targets) */
     int32_t reorder_every = 4, steps_to_reorder = 0; /* cell-order permutation interval, steps left */
     /* implicit particle tracking */
     fjsph_ipt_settings ipt{};
@@ -731,12 +731,17 @@ void group_blocks(fjsph_ctx* ctx)
  * fastest for large sets; below a few hundred thousand particles it leaves
  * too few blocks for 256 CUs, and blocks of 128 and 64, whose waves share
  * the lists (Split), win although they stage more.  ms a step with 256 / 128
- * / 64 targets, 3D: 100k Runge-Kutta 3.15 / 2.33 / 2.24, 268k 11.3 / 9.9 /
- * 9.7, 700k 7.83 / 7.76 / 9.00, 1M 12.6 / 12.7 / 15.2.  In 2D a target has
- * a tenth of the neighbours, so blocks are shorter work and the line lies
- * lower: 23k 0.98 / 0.96 / 0.91, 92k 1.14 / 1.17 / 1.26, 345k 1.80 / 2.08 /
- * 2.59.  FP64 keeps its blocks, see
- * block_shape. */
+ * / 64 targets, 3D: 100k Runge-Kutta 3.15 / 2.33 / 2.24, jets with ALE 220k
+ * 4.54 / 4.06 / 4.07, 300k 5.58 / 4.98 / 5.22, 400k 6.54 / 6.00 / 6.62, 549k
+ * 8.22 / 7.73 / 8.75, 700k 7.83 / 7.76 / 9.00, 1M 12.6 / 12.7 / 15.2;
+ * droplets, which iterate longer on the same lists, 113k 8.01 / 5.78 / 4.64,
+ * 195k 9.13 / 7.78 / 7.21, 268k 11.3 / 9.86 / 9.63.  The lower line lies where
+ * jets change over; a droplet just above it forgoes 2%.  In 2D a target has a
+ * tenth of the neighbours, so blocks are shorter work and the line lies
+ * lower: 6.5k 0.64 / 0.63 / 0.61, 12k 0.65 / 0.65 / 0.63, 23k 0.68 / 0.68 /
+ * 0.68, 35k 0.70 / 0.71 / 0.73, 55k 0.79 / 0.79 / 0.86, 92k 1.14 / 1.17 /
+ * 1.26, 345k 1.80 / 2.08 / 2.59; for the 4% of 64 targets below 20k there is
+ * no third line.  FP64 keeps its blocks, see block_shape. */
 int32_t default_targets(int dim, int64_t n, bool f32)
 {
     if (!f32) return 256;
@@ -2666,7 +2671,9 @@ fjsph_status fjsph_set_reorder_interval(fjsph_ctx* ctx, int32_t steps)
 fjsph_status fjsph_get_block_targets(fjsph_ctx* ctx, int32_t* targets)
 {
     if (!ctx || !targets) return FJSPH_ERR_ARG;
-    *targets = ctx->block_targets > 0 ? ctx->block_targets : 256;
+    *targets = ctx->block_targets > 0 ? ctx->block_targets
+               : ctx->have_state ? default_targets(ctx->s.dim, ctx->n, ctx->nl.f32 != 0)
+                                 : 256;
     return FJSPH_OK;
 }
 

@@ -247,7 +247,7 @@ class Engine:
         self._chk(self.lib.fjsph_get_block_targets(self.h, _ptr(t, _I32)), "get_block_targets")
         return int(t[0])
 
-    def autotune_blocks(self, candidates=(128, 192, 256, 384, 512), reps=3):
+    def autotune_blocks(self, candidates=(64, 128, 192, 256, 384, 512), reps=3):
         """fjsph_autotune_blocks: (best targets per block, {candidate: ms})."""
         c = np.ascontiguousarray(candidates, np.int32)
         ms = np.zeros(c.size)

@@ -367,15 +367,17 @@ fjsph_status fjsph_set_groups(fjsph_ctx* ctx, int32_t n_groups, const int32_t* g
  * step (out: count records). */
 fjsph_status fjsph_get_group_info(fjsph_ctx* ctx, int32_t first, int32_t count, fjsph_step_info* out);
 
-/* Targets per tile block of the pair passes (the cells of one block row
- * whose particles share one candidate union in LDS); 0 restores the
- * default: 256, or in mixed precision 128 or 64 while the particle set is
- * too small to fill the device with blocks of 256 (reported as 256).  No
+/* Targets per tile block of the pair passes (a box of cells whose particles
+ * share one candidate union in LDS); 0 restores the default: 256, or in
+ * mixed precision 128 or 64 while the particle set is too small to fill the
+ * device with blocks of 256.  fjsph_get_block_targets returns the number in
+ * use: the setting, or the default for the present particle set (256 before
+ * one is uploaded), so that setting what it returned changes nothing.  No
  * counterpart in the reference.  Results change only in the order of
- * summation.  A block spans at most 256 cells whatever the
- * setting, and a block whose candidate union overflows the 16-bit list
- * entries (a clustered region) makes the build halve the block length
- * and try again, down to one cell. */
+ * summation.  A block spans at most 256 cells along x whatever the setting,
+ * and a block whose candidate union overflows the 16-bit list entries (a
+ * clustered region) makes the build halve the block's longest side and try
+ * again, down to one cell. */
 fjsph_status fjsph_set_block_targets(fjsph_ctx* ctx, int32_t targets);
 fjsph_status fjsph_get_block_targets(fjsph_ctx* ctx, int32_t* targets);
 /* The first list build of a step moves the particles into cell order

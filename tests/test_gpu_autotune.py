@@ -101,3 +101,26 @@ def test_autotune_on_a_dynamic_inlet_matches_a_fresh_run():
         assert a.n == b.n
     for f in FIELDS:
         assert np.array_equal(a.field(f), b.field(f)), f
+
+
+@pytest.mark.parametrize("precision", [abi.PREC_MIXED, abi.PREC_FP64], ids=["mixed", "fp64"])
+def test_the_reported_setting_is_the_one_in_use(precision):
+    """Setting the reported number of targets changes nothing, and a small
+    set's default is among the candidates the autotuner tries by default."""
+    import inspect
+
+    from fjsph_amd.engine import Engine
+    case = cases.droplet_3d(diameter=1.0e-3, precision=precision)
+    print(f"[block targets] {case.n} particles precision={precision}", flush=True)
+    a, b = Engine(case), Engine(case)
+    got = b.get_block_targets()
+    b.set_block_targets(got)
+    assert b.get_block_targets() == got
+    for e in (a, b):
+        e.integrate_no_update()
+    for _ in range(2):
+        assert a.integrate_step() == b.integrate_step()
+    for f in FIELDS:
+        assert np.array_equal(a.field(f), b.field(f)), f
+    assert a.get_block_targets() == got
+    assert got in inspect.signature(Engine.autotune_blocks).parameters["candidates"].default
