@@ -403,6 +403,7 @@ void alloc_slots(fjsph_ctx* ctx, int64_t cap, int64_t keep)
 {
     const size_t D = size_t(ctx->s.dim), c = size_t(cap), k = size_t(keep);
     HIPCHK(hipStreamSynchronize(ctx->st));
+    free_spare(ctx); /* of the old size; a set too large for it takes none again */
     for (DevState* st : {&ctx->pn, &ctx->pnp1}) {
         for (int f = 0; f < kNumFields; ++f) {
             void** slot = field_slot(*st, f);

@@ -45,3 +45,32 @@ def test_state_copy(n):
     for f in abi.F:
         assert np.array_equal(eng.field(f, abi.STATE_N), eng.field(f, abi.STATE_NP1)), f
     eng.close()
+
+
+def test_a_growing_set_gives_its_spare_state_back():
+    """Small sets keep buffers for a whole state's reordering; a set that
+    grows past the size up to which they are used frees them.  They are more
+    than the growth of everything else here, so the context shrinks."""
+    import ctypes as C
+    case = cases.pipe_inlet_3d(diameter=9.1e-3, dx=5e-5, mode=0, precision=abi.PREC_MIXED, exit_to_delete=100.0)
+    print(f"[fields] growing set n={case.n}", flush=True)
+    assert case.n < 300_000
+    eng = _engine(case)
+    eng.set_reorder_interval(1)
+    eng.integrate_no_update()
+    eng.integrate_step()
+
+    def free():
+        b, total = C.c_size_t(), C.c_size_t()
+        assert eng.lib.hipMemGetInfo(C.byref(b), C.byref(total)) == 0
+        return b.value
+
+    before = free()
+    for _ in range(30):
+        eng.integrate_step()
+        if eng.n > case.n:
+            break
+    assert eng.n > 300_000
+    eng.integrate_step()
+    assert free() > before
+    eng.close()
