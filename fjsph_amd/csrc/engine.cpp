@@ -3349,7 +3349,7 @@ fjsph_status fjsph_surrogate_grad(fjsph_ctx* ctx, int32_t n_hidden, int32_t batc
         m.idx = didx;
         mlp_params(m, p, wf, wt);
         launch_mlp_pack(D, p, L, wf, wt, ctx->st);
-        launch_mlp_train(D, m, ctx->st);
+        HIPCHK(launch_mlp_train(D, m, ctx->st));
         launch_mlp_reduce(m, g, g + m.nw, sse, ctx->st);
         sync(ctx);
         HIPCHK(hipMemcpy(dweights, g, size_t(m.nw) * 4, hipMemcpyDeviceToHost));
@@ -3410,7 +3410,7 @@ fjsph_status fjsph_surrogate_grad_noalloc(fjsph_ctx* ctx, int32_t n_hidden, int3
         m.wt = wt;
         m.b = biases;
         m.bo = biases + int64_t(L) * 64;
-        launch_mlp_train(D, m, ctx->st);
+        HIPCHK(launch_mlp_train(D, m, ctx->st));
         launch_mlp_reduce(m, dweights, dbiases, loss ? sse : nullptr, ctx->st);
         if (loss) launch_mlp_loss(sse, double(batch) * NO, loss, ctx->st);
         sync(ctx);
@@ -3467,7 +3467,7 @@ fjsph_status fjsph_surrogate_train(fjsph_ctx* ctx, int64_t n, const double* poin
         const double b1 = 0.9, b2 = 0.999;
         for (int32_t t = 1; t <= steps; ++t) {
             launch_mlp_pack_draw(D, p, L, wf, wt, seed, t, n, batch, didx, ctx->st);
-            launch_mlp_train(D, m, ctx->st);
+            HIPCHK(launch_mlp_train(D, m, ctx->st));
             const double lr_t = lr * 0.5 * (1.0 + std::cos(3.14159265358979323846 * double(t - 1) / double(steps)));
             launch_mlp_reduce_adam(m, sse + (t - 1),
                                    MlpAdam{p, m1, m2, float(lr_t), float(b1), float(b2), 1e-8f,

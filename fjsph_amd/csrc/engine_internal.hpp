@@ -374,7 +374,7 @@ void launch_delete_flag(int dim, DevState s, const int32_t* part_id, const int32
                         int64_t n_bound, int32_t* keep, int32_t* hflag, int32_t* blkcount, hipStream_t st);
 void launch_compact_perm(const int32_t* keep, const int32_t* start, int64_t n, int32_t* perm, hipStream_t st);
 void launch_compact_ids(int32_t* part_id, const int32_t* hstart, int64_t n, hipStream_t st);
-void launch_mlp_train(int dim, const MlpTrain& m, hipStream_t st);
+[[nodiscard]] hipError_t launch_mlp_train(int dim, const MlpTrain& m, hipStream_t st);
 /* Sums of the per-block partials: the gradients of the weights and biases,
  * the squared error into *sse (null: not wanted). */
 void launch_mlp_reduce(const MlpTrain& m, float* gw, float* gb, float* sse, hipStream_t st);

@@ -400,16 +400,20 @@ __global__ __launch_bounds__(TPB) void k_mlp_pack(const float* __restrict__ w, i
     }
 }
 
-void launch_mlp_train(int dim, const MlpTrain& m, hipStream_t st)
+hipError_t launch_mlp_train(int dim, const MlpTrain& m, hipStream_t st)
 {
     const dim3 g((unsigned)(m.batch / 64)), b(TPB);
     const size_t lds = size_t(train_lds(m.n_hidden)) * sizeof(__bf16);
     const auto k = dim == 2 ? k_mlp_train<2> : k_mlp_train<3>;
     /* more than the default 64 KiB from five hidden layers on */
-    if (lds > 65536)
-        (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  int(train_lds(8) * sizeof(__bf16)));
-    hipLaunchKernelGGL(k, g, b, lds, st, m);
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 int(train_lds(8) * sizeof(__bf16)));
+        if (e != hipSuccess) return e;
+    }
+    MlpTrain arg = m;
+    void* args[] = {&arg};
+    return hipLaunchKernel((const void*)k, g, b, args, lds, st);
 }
 
 void launch_mlp_reduce(const MlpTrain& m, float* gw, float* gb, float* sse, hipStream_t st)
