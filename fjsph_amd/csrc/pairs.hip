@@ -3085,10 +3085,13 @@ void launch_boundary(int dim, const Consts& c, DevState s, Aux a, const int32_t*
                      TileGrid tg, NbrList nl, int64_t n, int64_t nb, int32_t* slots, bool listed, int32_t* near_inlet,
                      hipStream_t st)
 {
-    /* the block's slots (at most nb, the boundary count), listed once for an
-     * order of the slots, then one wave each: with Aux kept up by k_bnd_solve
-     * a sub-iteration has three launches of 5-8 us fewer (6.5k particles 1.17
-     * -> 1.02 ms a step, of which the FP64 dSPH pass 0.01) */
+    /* the block's slots (at most nb, the boundary count), then one wave each.
+     * Of one wall block they are listed once for an order of the slots; with
+     * several each takes the other's place, and all are listed every time.
+     * With Aux kept up by k_bnd_solve a sub-iteration has three launches of
+     * 5-8 us fewer (6.5k particles, one block: 1.17 -> 1.02 ms a step, of
+     * which the FP64 dSPH pass 0.01), and a block reads the volumes that an
+     * Adami block before it has set, as the sequential solvers do */
     if (!listed) {
         hipLaunchKernelGGL(k_clear_count, dim3(1), dim3(1), 0, st, slots);
         hipLaunchKernelGGL(k_block_slots, dim3(grid_of(n)), dim3(TPB), 0, st, blk, n, block, slots);

@@ -6,6 +6,7 @@ counts and rollbacks equal):
   - DBC walls (src/Resid.cpp:21-76): the dam break and a 3D walled block;
   - ghost walls (src/Resid.cpp:78-141), free-slip and no-slip
     (Set_No_Slip, src/Resid.cpp:143-186), 2D and 3D, Newmark-Beta and RK4;
+  - two wall blocks with different solvers, in either order;
   - a wall moving by a velocity table (src/Newmark_Beta.cpp:69-84);
   - a ghost wall particle next to BUFFER fluid, whose density is clamped
     near the inlet (src/Newmark_Beta.cpp:163-178);
@@ -18,6 +19,7 @@ import pytest
 
 from fjsph_amd import abi, cases
 from tests.parity import assert_close
+from tests.test_gpu_parity import MIXED_STEP
 
 pytestmark = pytest.mark.gpu
 
@@ -123,6 +125,43 @@ def test_boundary_solver_steps_rk4(name, make):
         assert abs(ie["dt"] - io["dt"]) <= 1e-10 * io["dt"]
     for f in ("X", "V", "RHO", "P", "ACC", "RRHO"):
         assert_close(f, eng.field(f), orc.field(f), FP64_STEP)
+    eng.close()
+
+
+@pytest.mark.parametrize("precision", [abi.PREC_FP64, abi.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("integrator", [abi.NEWMARK_BETA, abi.RUNGE_KUTTA], ids=["nb", "rk4"])
+@pytest.mark.parametrize("solvers", [(abi.PRESSURE_G, abi.GHOST), (abi.GHOST, abi.PRESSURE_G)],
+                         ids=["adami-ghost", "ghost-adami"])
+def test_two_wall_blocks(solvers, integrator, precision):
+    """Two wall blocks with different solvers, every other wall particle in
+    each and with a velocity of its own, so that each block enters the
+    other's sums.  They are solved in turn: a ghost particle's density rate
+    is of the volumes that an Adami block before it has just set."""
+    case = _dam(solvers[0], seed=14)
+    nb = case.n_bound
+    order = np.r_[0:nb:2, 1:nb:2, nb:case.n]
+    for f in ("x", "v", "rho", "p", "m", "b"):
+        setattr(case, f, np.ascontiguousarray(getattr(case, f)[order]))
+    half = (nb + 1) // 2
+    wall = case.blocks[0]
+    case.blocks = [dict(wall, last=half, vel=(0.5, 0.0, 0.0)),
+                   dict(wall, first=half, bound_solver=solvers[1], vel=(0.0, 0.5, 0.0))] + case.blocks[1:]
+    case.settings.integrator, case.settings.precision = integrator, precision
+    print(f"[two walls] {solvers} integrator={integrator} precision={precision} n={case.n} nb={nb}", flush=True)
+    eng, orc = _pair(case)
+    eng.integrate_no_update()
+    orc.integrate_no_update()
+    fp64 = precision == abi.PREC_FP64
+    for _ in range(4 if fp64 else 1):
+        ie, io = eng.integrate_step(), orc.integrate_step()
+        if fp64:
+            assert ie["iterations"] == io["iterations"]
+        assert abs(ie["dt"] - io["dt"]) <= (1e-10 if fp64 else MIXED_STEP) * io["dt"]
+    tol = FP64_STEP if fp64 else MIXED_STEP
+    for f in ("X", "V", "RHO", "P", "ACC", "RRHO"):
+        assert_close(f, eng.field(f), orc.field(f), tol)
+    for f in ("RHO", "RRHO"):
+        assert_close(f + "_wall", eng.field(f)[:nb], orc.field(f)[:nb], tol)
     eng.close()
 
 
