@@ -157,3 +157,28 @@ def test_cell_scan(cells):
     off_o, idx_o, _ = orc.neighbours()
     assert same_neighbour_sets(off_e, idx_e, off_o, idx_o)
     eng.close()
+
+
+@pytest.mark.parametrize("cells", [2048 * 1024, 2048 * 1024 + 1, 2048 * 1300 + 77])
+def test_cell_scan_of_many_tiles(cells):
+    """The same over a row of more cells than tiles' sums are added up
+    directly for (1024 tiles): the last such size, one tile more, and a
+    number of tiles and of cells in the last that are no multiples of
+    anything.  One particle to four cells, the sparsest grid there may be."""
+    c = _clusters(2, (13,), abi.PREC_FP64, 0)
+    dx, n = c.settings.particle_step, cells // 4
+    cs = 4 * dx * (1.0 + 1e-7)
+    rng = np.random.default_rng(31)
+    c.x = np.stack([rng.uniform(0.0, (cells - 1) * cs, n), rng.uniform(0.0, 0.5 * cs, n)], 1)
+    c.x[7], c.x[n // 2] = 0.0, ((cells - 0.9) * cs, 0.0)
+    c.v, c.rho, c.p = np.zeros((n, 2)), np.full(n, c.settings.rho_rest), np.zeros(n)
+    c.m, c.b = np.full(n, c.settings.rho_rest * dx ** 2), np.full(n, abi.FREE, dtype=np.int32)
+    c.blocks = [dict(first=0, last=n, is_fluid=1)]
+    print(f"[walk] scan of {cells} cells n={n}", flush=True)
+    eng, orc = _engine(c), _oracle(c)
+    eng.build_neighbours()
+    orc.build_neighbours()
+    off_e, idx_e = eng.neighbours()
+    off_o, idx_o, _ = orc.neighbours()
+    assert same_neighbour_sets(off_e, idx_e, off_o, idx_o)
+    eng.close()
