@@ -86,13 +86,14 @@ def workload(name, n_target):
 def load_traffic(n):
     """HBM bytes per k_force_m launch from the committed rocprofv3 --pmc
     summary (FETCH_SIZE + WRITE_SIZE, scaled by the copy-kernel factor),
-    rescaled to n particles."""
+    rescaled to n particles, and the rate at which the counted launches
+    moved theirs (GB/s)."""
     try:
         with open(TRAFFIC_FILE) as f:
             t = json.load(f)
-        return t["bytes_per_particle"] * n, t
+        return t["bytes_per_particle"] * n, t["bytes_per_launch"] / t["ms_per_launch"] / 1e6, t
     except (OSError, ValueError, KeyError):
-        return None, None
+        return None, None, None
 
 
 def cpu_baseline(args):
@@ -407,13 +408,14 @@ def main():
     avg_s = (ms / 1e3) / max(launches, 1)
     bpp = run["force_bpp"]
     achieved_gbs = bpp * case.n / avg_s / 1e9
-    traffic, tmeta = load_traffic(case.n)
+    traffic, traffic_rate, tmeta = load_traffic(case.n)
     fpp = force_flops_per_pair(case.settings.dim, bool(case.settings.ale))
     tflops = fpp * pairs / avg_s / 1e12
     hbm = {"achieved": achieved_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved_gbs / HBM_PEAK_GBS,
            "alg_bytes_per_particle": bpp, "traffic": traffic,
            "traffic_source": os.path.relpath(TRAFFIC_FILE, ROOT) if tmeta else None,
-           "traffic_rate_GBs": traffic / avg_s / 1e9 if traffic else None}
+           # over the counted launches' own time, not this run's
+           "traffic_rate_GBs": traffic_rate}
     valu = {"achieved": tflops, "peak": FP32_VECTOR_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": tflops / FP32_VECTOR_PEAK_TFLOPS,
             # the published FP32 peak counts packed (2-wide) FP32; the engine is built without packed
