@@ -756,8 +756,7 @@ int32_t default_targets(int dim, int64_t n, bool f32)
  * need 48, and of a 2D block of 38 cells 120 or, as 6 x 6, 64 (345k
  * particles: 2.39 -> 2.04 ms a step; 1M jet 14.5 -> 14.3, 1M jet in
  * crossflow 21.5 -> 20.7, 256 drops 30.7 -> 29.4).  The rows of the union keep to kMaxRows, so a
- * long block grows along x, up to kMaxBlockCells cells (the list build's
- * FP32 prefilter band holds up to that length).  Independent simulations
+ * long block grows along x, up to kMaxBlockCells cells.  Independent simulations
  * are stacked along the last axis one empty layer apart, so that their
  * blocks stay one layer thick.  In FP64 the blocks are rows of cells for
  * about 256 targets whatever the particle count: the order of every sum

@@ -71,9 +71,9 @@ constexpr uint32_t NO_ENTRY = 0xFFFF;
 constexpr int kRowSlack = 4;
 /* Cell rows of a block's candidate union at most. */
 constexpr int kMaxRows = 25;
-/* Longest tile block in cells: every coordinate of a block's candidate
- * union then lies within 1000 H of its first target, the bound the FP32
- * prefilter of the list build relies on. */
+/* Cells of a tile block along x at most: the FP32 coordinates relative to
+ * its first target then stay within about 500 H (the list build's band, in
+ * which the FP64 test decides, follows the block's extent). */
 constexpr int32_t kMaxBlockCells = 256;
 
 /* Tile decomposition of the last neighbour build: the blocks are boxes of

@@ -1036,7 +1036,8 @@ __global__ __launch_bounds__(PTPB) void k_dsph_t(Consts c, DevState s, Aux ax, T
  * (dsph_pair), so the rank test of its correction matrix, which decides
  * between L^-1 and the identity, sees the matrix of the FP64 path.
  *
- * Four waves per SIMD: the two pairs' terms fit their 128 registers, while a
+ * Four waves per SIMD: the two pairs' terms all but fit their 128 registers
+ * (8 B a lane spilled in 3D, 20 B with build positions), while a
  * fifth wave spilled 112 B a lane into the pair loop (the whole pass: 268k
  * particles 0.267 -> 0.243 ms, 700k 0.563 -> 0.499, 4M 2.60 -> 2.32).  The surface
  * loops do better with five, spilling as they do (268k 0.582 ms together,
